@@ -398,8 +398,14 @@ __global__ __launch_bounds__(256) void k_block_ops(BlockOpArgs a) {
           double uu = u0 * u0;
           uu += u1 * u1;
           uu += u2 * u2;
+          const double du = over_cs2x2(uu);
+          f[REST] -= a.omega * (f[REST] - W64(REST) * rho * (1.0 - du));
 #pragma unroll
-          for (int q = 0; q < Q; q++) f[q] -= a.omega * (f[q] - feq_f64(q, rho, u0, u1, u2, uu));
+          for (int q = 0; q < REST; q++) {
+            const FeqPair e = feq_pair_f64(q, rho, cdot64(q, u0, u1, u2), du);
+            f[q] -= a.omega * (f[q] - e.q);
+            f[Q - 1 - q] -= a.omega * (f[Q - 1 - q] - e.mirror);
+          }
         }
       }
     }

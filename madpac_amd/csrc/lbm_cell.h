@@ -80,6 +80,31 @@ __device__ __forceinline__ double cdot64(int q, double v0, double v1, double v2)
   return r;
 }
 
+// Divisions by the constants of computeFeq (BLB/BlockComputeCellValues.cpp:14-20): c = 1.0/3.0,
+// 2.0*(1.0/3.0) and 2.0*(1.0/3.0)*(1.0/3.0), each rounded to double.  x / c = fma(z, x, zl * x) to the
+// last bit, where z + zl is 1/c to twice the precision (the method of Brisebarre, Muller and Raina,
+// IEEE Trans. Computers 53(8), 2004).  All three c are z^-1 (1 - 2^-54) up to 2^-108, so z = 3, 1.5, 4.5
+// and zl = z 2^-54, and the sum before its one rounding is within 0.75 2^-106 of the quotient, relative;
+// no quotient of two doubles by these c lies that close to a rounding boundary (a midpoint quotient
+// m/2 would need |2^53 X - m C| < 1 for odd integers m, C (< 4 where 4 divides C): never).  Zeros,
+// infinities, NaN and overflow follow the division; below 2^-960 the last bit may not, and every
+// caller adds the result to 1.  Two FP64 instructions each; the compiler's division takes ten and a
+// quarter-rate reciprocal, and 40 of them made a cell's collision 675 instructions instead of 270.
+__device__ __forceinline__ double over_cs2(double x) { return __builtin_fma(3.0, x, x * 0x1.8p-53); }
+__device__ __forceinline__ double over_cs2x2(double x) { return __builtin_fma(1.5, x, x * 0x1.8p-54); }
+__device__ __forceinline__ double over_cs4x2(double x) { return __builtin_fma(4.5, x, x * 0x1.2p-52); }
+
+// computeFeq (BLB/BlockComputeCellValues.cpp:14-20) of direction q (cu = c_q . u, du = u.u / (2 cs2))
+// and of its mirror 18 - q, whose c . u is -cu and whose weight is the same: cu / cs2 changes its sign
+// and cu^2 / (2 cs4) is shared, exactly.
+struct FeqPair {
+  double q, mirror;
+};
+__device__ __forceinline__ FeqPair feq_pair_f64(int q, double rho, double cu, double du) {
+  const double a = over_cs2(cu), b = over_cs4x2(cu * cu), wr = W64(q) * rho;
+  return FeqPair{wr * (1.0 + a + b - du), wr * (1.0 - a + b - du)};
+}
+
 // ---------------------------------------------------------------------------------------------
 // FP64, reference operation order.  f[] in, post-collision f*[] out (in place).  Returns rho.
 // FORCE: Guo forcing with equilibrium velocity u + g/2.  ALPHA: equilibrium velocity scaled by
@@ -120,17 +145,17 @@ __device__ __forceinline__ double collide_f64(double (&f)[Q], const CollideParam
     u1 = (1.0 - alpha) * u1;
     u2 = (1.0 - alpha) * u2;
   }
-  // computeFeq (:14-20) and BGK (BlockBGK.cpp:43)
+  // computeFeq (:14-20) and BGK (BlockBGK.cpp:43), a direction and its mirror together
   double uu = u0 * u0;
   uu += u1 * u1;
   uu += u2 * u2;
-  const double omega = p.omega;
+  const double omega = p.omega, du = over_cs2x2(uu);
+  f[REST] -= omega * (f[REST] - W64(REST) * rho * (1.0 - du));
 #pragma unroll
-  for (int q = 0; q < Q; q++) {
-    const double cu = cdot64(q, u0, u1, u2);
-    const double feq = W64(q) * rho *
-        (1.0 + cu / (1.0 / 3.0) + (cu * cu) / (2.0 * (1.0 / 3.0) * (1.0 / 3.0)) - (uu / (2.0 * (1.0 / 3.0))));
-    f[q] -= omega * (f[q] - feq);
+  for (int q = 0; q < REST; q++) {
+    const FeqPair e = feq_pair_f64(q, rho, cdot64(q, u0, u1, u2), du);
+    f[q] -= omega * (f[q] - e.q);
+    f[Q - 1 - q] -= omega * (f[Q - 1 - q] - e.mirror);
   }
   if (FORCE) {
     // Guo source (1 - 1/(2 tau)) w rho [3 (c - u).g + 9 (c.u)(c.g)] with cs2 = 1/3 folded into the
@@ -139,11 +164,14 @@ __device__ __forceinline__ double collide_f64(double (&f)[Q], const CollideParam
     double ug = u0 * p.g[0];
     ug += u1 * p.g[1];
     ug += u2 * p.g[2];
+    f[REST] += pref * W64(REST) * (3.0 * (0.0 - ug));
 #pragma unroll
-    for (int q = 0; q < Q; q++) {
+    for (int q = 0; q < REST; q++) {
       const double cu = cdot64(q, u0, u1, u2);
       const double cg = cdot64(q, p.g[0], p.g[1], p.g[2]);
-      f[q] += pref * W64(q) * (3.0 * (cg - ug) + 9.0 * cu * cg);
+      const double quad = 9.0 * cu * cg;  // the same for the mirror direction
+      f[q] += pref * W64(q) * (3.0 * (cg - ug) + quad);
+      f[Q - 1 - q] += pref * W64(q) * (3.0 * (-cg - ug) + quad);
     }
   }
   return rho;
@@ -255,17 +283,23 @@ __device__ __forceinline__ float collide_f32s_h(float (&gs)[Q], const CollidePar
   const double uu15 = 1.5 * (u0 * u0 + u1 * u1 + u2 * u2);
   const float rho32 = (float)rho, v0 = (float)u0, v1 = (float)u1, v2 = (float)u2;
   const float ug = FORCE ? v0 * p32.g[0] + v1 * p32.g[1] + v2 * p32.g[2] : 0.f;
-#pragma unroll
-  for (int q = 0; q < Q; q++) {
-    const double cu = cdot64(q, u0, u1, u2);
-    const float geq = (float)(W64(q) * (drho + rho * (3.0 * cu + 4.5 * cu * cu - uu15)));
+  // one population: relax toward geq, then the force term with its (c.u)(c.g) part given
+  auto relax = [&](int q, double lin, float cg, float quad) {
+    const float geq = (float)(W64(q) * (drho + rho * lin));
     float v = gs[q] - (float)(p.omega * (double)(gs[q] - geq));
-    if (FORCE) {
-      const float cg = (float)CX(q) * p32.g[0] + (float)CY(q) * p32.g[1] + (float)CZ(q) * p32.g[2];
-      const float cuf = (float)cu;
-      v += p32.fpref * W32(q) * rho32 * (3.0f * (cg - ug) + 9.0f * cuf * cg);
-    }
+    if (FORCE) v += p32.fpref * W32(q) * rho32 * (3.0f * (cg - ug) + quad);
     gs[q] = v;
+  };
+  relax(REST, 0.0 - uu15, 0.f, 0.f);
+#pragma unroll
+  for (int q = 0; q < REST; q++) {
+    // a direction and its mirror: c.u and c.g change sign, the quadratic terms are shared (exactly)
+    const double cu = cdot64(q, u0, u1, u2);
+    const double a = 3.0 * cu, b = 4.5 * cu * cu;
+    const float cg = FORCE ? (float)CX(q) * p32.g[0] + (float)CY(q) * p32.g[1] + (float)CZ(q) * p32.g[2] : 0.f;
+    const float quad = FORCE ? 9.0f * (float)cu * cg : 0.f;
+    relax(q, a + b - uu15, cg, quad);
+    relax(Q - 1 - q, -a + b - uu15, -cg, quad);
   }
   return rho32;
 }
@@ -286,8 +320,7 @@ __device__ __forceinline__ float moving_wall_f32(int q, const double* uw, float 
 // computeFeq (BLB/BlockComputeCellValues.cpp:14-20) for one direction, reference order:
 __device__ __forceinline__ double feq_f64(int q, double rho, double u0, double u1, double u2, double uu) {
   const double cu = cdot64(q, u0, u1, u2);
-  return W64(q) * rho *
-         (1.0 + cu / (1.0 / 3.0) + (cu * cu) / (2.0 * (1.0 / 3.0) * (1.0 / 3.0)) - (uu / (2.0 * (1.0 / 3.0))));
+  return W64(q) * rho * (1.0 + over_cs2(cu) + over_cs4x2(cu * cu) - over_cs2x2(uu));
 }
 
 // (the cell velocity comes by value: a pointer select between it and the table would force it

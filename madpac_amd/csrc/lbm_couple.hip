@@ -77,8 +77,14 @@ __device__ __forceinline__ double collide_coupled_f64(double (&f)[Q], const Coup
   double uu = u[0] * u[0];
   uu += u[1] * u[1];
   uu += u[2] * u[2];
+  const double du = over_cs2x2(uu);
+  f[REST] -= a.omega * (f[REST] - W64(REST) * rho * (1.0 - du));
 #pragma unroll
-  for (int q = 0; q < Q; q++) f[q] -= a.omega * (f[q] - feq_f64(q, rho, u[0], u[1], u[2], uu));
+  for (int q = 0; q < REST; q++) {
+    const FeqPair e = feq_pair_f64(q, rho, cdot64(q, u[0], u[1], u[2]), du);
+    f[q] -= a.omega * (f[q] - e.q);
+    f[Q - 1 - q] -= a.omega * (f[Q - 1 - q] - e.mirror);
+  }
   if (dir) {
     // adjustF / computeGi, with (c.u)^2 as the reference writes it
     const double pref = 1.0 - 0.5 / a.tau;

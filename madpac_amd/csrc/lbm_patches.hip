@@ -391,9 +391,7 @@ __global__ __launch_bounds__(256) void k_patch_init(const PatchDev* __restrict__
     uu += u2 * u2;
 #pragma unroll
     for (int q = 0; q < Q; q++) {
-      const double cu = cdot64(q, u0, u1, u2);
-      const double feq = W64(q) * r *
-          (1.0 + cu / (1.0 / 3.0) + (cu * cu) / (2.0 * (1.0 / 3.0) * (1.0 / 3.0)) - (uu / (2.0 * (1.0 / 3.0))));
+      const double feq = feq_f64(q, r, u0, u1, u2, uu);
       const T v = (sizeof(T) == 8) ? (T)feq : (T)(feq - W64(q));
       s[base + ref_slot(q, n, x, y, z, c, w)] = v;
     }
