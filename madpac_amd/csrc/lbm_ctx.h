@@ -78,7 +78,8 @@ struct lbm_ctx {
 };
 
 double lbm_tau_effective(double tau);
-int lbm_enqueue_steps(lbm_ctx* c, int nsteps);
+// nsteps steps of the current state, two per launch where that is faster unless `single`
+int lbm_enqueue_steps(lbm_ctx* c, int nsteps, bool single = false);
 // the geometry with the layout of the current stored state (for the reading/writing kernels)
 inline lbm::DenseGeom lbm_state_geom(const lbm_ctx* c) {
   lbm::DenseGeom g = c->g;

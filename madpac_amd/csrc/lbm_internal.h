@@ -126,6 +126,17 @@ hipError_t launch_dense_step(const DenseGeom& g, bool fp32, bool f32math, const 
                              const uint32_t* words,
                              const void* alpha, bool force, bool walls, const CollideParams& p64,
                              const CollideParams32& p32, const BoundaryArgs& bc, bool spec, hipStream_t stream);
+// Two steps src -> dst in one launch (lbm_pair.hip): the same state as two launch_dense_step.
+struct PairGeom {
+  int tx, ty, tz;  // tiles of columns along x and y, chunks along z
+  int cz;          // planes per chunk
+  int64_t nblocks, nblocks_padded;
+};
+// whether launch_dense_pair takes this lattice and is the faster way
+bool pair_fits(const DenseGeom& g, size_t esize, bool walls);
+hipError_t launch_dense_pair(const DenseGeom& g, bool fp32, bool f32math, const void* src, void* dst,
+                             const uint32_t* words, const void* alpha, bool force, bool walls, const CollideParams& p64,
+                             const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t stream);
 // reference state f (FP64) from the stored state
 // one in-place AA step on a single buffer: parity 0 reads the NATURAL layout and leaves SWAPPED,
 // parity 1 the reverse
