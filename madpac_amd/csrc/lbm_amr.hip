@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "lbm_blockstore.h"
+#include "lbm_readout.h"
 
 namespace lbm {
 
@@ -250,6 +251,7 @@ int lbm_blocks_create(lbm_blockstore** out, int64_t nblocks, int device) {
   if (!out) return LBM_ERR_ARG;
   *out = nullptr;
   lbm_blockstore* bs = new lbm_blockstore();
+  lbm::readout_hold();
   auto bail = [&](int code, const std::string& m) {
     g_blocks_create_error = m;
     lbm_blocks_destroy(bs);
@@ -289,6 +291,7 @@ int lbm_blocks_destroy(lbm_blockstore* bs) {
   if (bs->ev0) (void)hipEventDestroy(bs->ev0);
   if (bs->ev1) (void)hipEventDestroy(bs->ev1);
   if (bs->stream) (void)hipStreamDestroy(bs->stream);
+  lbm::readout_release();
   delete bs;
   return LBM_OK;
 }
@@ -316,15 +319,12 @@ int lbm_blocks_get(lbm_blockstore* bs, int64_t first, int64_t count, double* pdf
   if (!bs) return LBM_ERR_ARG;
   if (int rc = check_range(bs, first, count)) return rc;
   BCHK(bs, hipSetDevice(bs->device));
-  if (pdf)
-    BCHK(bs, hipMemcpyAsync(pdf, bs->pdf + first * BP, (size_t)count * BP * sizeof(double), hipMemcpyDeviceToHost, bs->stream));
-  if (density)
-    BCHK(bs, hipMemcpyAsync(density, bs->density + first * BC, (size_t)count * BC * sizeof(double), hipMemcpyDeviceToHost,
-                            bs->stream));
-  if (velocity)
-    BCHK(bs, hipMemcpyAsync(velocity, bs->velocity + first * BV, (size_t)count * BV * sizeof(double), hipMemcpyDeviceToHost,
-                            bs->stream));
-  BCHK(bs, hipStreamSynchronize(bs->stream));
+  lbm::HostCopy parts[3];
+  int n = 0;
+  if (pdf) parts[n++] = {pdf, bs->pdf + first * BP, (size_t)count * BP * sizeof(double)};
+  if (density) parts[n++] = {density, bs->density + first * BC, (size_t)count * BC * sizeof(double)};
+  if (velocity) parts[n++] = {velocity, bs->velocity + first * BV, (size_t)count * BV * sizeof(double)};
+  BCHK(bs, lbm::read_back(parts, n, bs->stream));
   return LBM_OK;
 }
 

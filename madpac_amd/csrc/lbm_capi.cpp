@@ -13,6 +13,7 @@
 
 #include "lbm_ctx.h"
 #include "lbm_internal.h"
+#include "lbm_readout.h"
 
 using lbm::Q;
 
@@ -153,6 +154,7 @@ int lbm_create(lbm_ctx** out, const lbm_config* cfg) {
   if (cfg->device < 0 || cfg->device >= ndev) return fail(nullptr, LBM_ERR_ARG, "device ordinal out of range");
 
   lbm_ctx* c = new lbm_ctx();
+  lbm::readout_hold();
   c->cfg = *cfg;
   c->fp32 = cfg->precision != LBM_FP64;
   c->f32math = cfg->precision == LBM_FP32_SHIFTED_F32;
@@ -220,6 +222,7 @@ int lbm_destroy(lbm_ctx* c) {
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  lbm::readout_release();
   delete c;
   return LBM_OK;
 }
@@ -478,8 +481,8 @@ int lbm_get_populations(lbm_ctx* c, double* f) {
   if (rc) return rc;
   HIPCHK(c, lbm::launch_dense_pull(lbm_state_geom(c), c->fp32, c->buf[c->cur], (double*)c->scratch, c->words,
                                    c->stream));
-  HIPCHK(c, hipMemcpyAsync(f, c->scratch, bytes, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  const lbm::HostCopy part{f, c->scratch, bytes};
+  HIPCHK(c, lbm::read_back(&part, 1, c->stream));
   return LBM_OK;
 }
 
@@ -738,9 +741,8 @@ int lbm_get_fields(lbm_ctx* c, double* rho, double* u) {
   double* d_rho = (double*)c->scratch;
   double* d_u = d_rho + n;
   HIPCHK(c, lbm::launch_dense_fields(lbm_state_geom(c), c->fp32, c->buf[c->cur], c->words, d_rho, d_u, c->stream));
-  HIPCHK(c, hipMemcpyAsync(rho, d_rho, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(u, d_u, 3 * n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  const lbm::HostCopy parts[2] = {{rho, d_rho, n * sizeof(double)}, {u, d_u, 3 * n * sizeof(double)}};
+  HIPCHK(c, lbm::read_back(parts, 2, c->stream));
   return LBM_OK;
 }
 

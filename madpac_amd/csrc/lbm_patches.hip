@@ -26,6 +26,7 @@
 #include "lbm_capi.h"
 #include "lbm_cell.h"
 #include "lbm_internal.h"
+#include "lbm_readout.h"
 
 namespace lbm {
 
@@ -678,6 +679,7 @@ int lbm_patches_create(lbm_patchset** out, const lbm_patch* table, int npatches,
   if (!out) return LBM_ERR_ARG;
   *out = nullptr;
   lbm_patchset* ps = new lbm_patchset();
+  lbm::readout_hold();
   auto bail = [&](int code, const std::string& m) {
     g_patch_create_error = m;  // lbm_patches_last_error(NULL) reports it
     lbm_patches_destroy(ps);
@@ -758,6 +760,7 @@ int lbm_patches_destroy(lbm_patchset* ps) {
   if (ps->ev0) (void)hipEventDestroy(ps->ev0);
   if (ps->ev1) (void)hipEventDestroy(ps->ev1);
   if (ps->stream) (void)hipStreamDestroy(ps->stream);
+  lbm::readout_release();
   delete ps;
   return LBM_OK;
 }
@@ -862,8 +865,8 @@ int lbm_patches_get_populations(lbm_patchset* ps, double* f) {
     hipLaunchKernelGGL(k_patch_pull<double>, grid, dim3(256), 0, ps->stream, ps->d_patches, (int)ps->host.size(),
                        ps->d_cell_base, ps->d_words, (const double*)ps->buf[ps->cur], d_f);
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(f, d_f, bytes, hipMemcpyDeviceToHost, ps->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ps->stream);
+  const lbm::HostCopy part{f, d_f, bytes};
+  if (e == hipSuccess) e = lbm::read_back(&part, 1, ps->stream);
   (void)hipFree(d_f);
   if (e != hipSuccess) return pfail(ps, LBM_ERR_HIP, std::string("patch readout: ") + hipGetErrorString(e));
   return LBM_OK;
@@ -891,9 +894,8 @@ int lbm_patches_get_fields(lbm_patchset* ps, double* rho, double* u) {
     hipLaunchKernelGGL(k_patch_fields<double>, grid, dim3(256), 0, ps->stream, ps->d_patches, (int)ps->host.size(),
                        ps->d_cell_base, ps->d_words, (const double*)ps->buf[ps->cur], d_rho, d_u);
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(rho, d_rho, cells * sizeof(double), hipMemcpyDeviceToHost, ps->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(u, d_u, 3 * cells * sizeof(double), hipMemcpyDeviceToHost, ps->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ps->stream);
+  const lbm::HostCopy parts[2] = {{rho, d_rho, cells * sizeof(double)}, {u, d_u, 3 * cells * sizeof(double)}};
+  if (e == hipSuccess) e = lbm::read_back(parts, 2, ps->stream);
   (void)hipFree(d_f);
   if (e != hipSuccess) return pfail(ps, LBM_ERR_HIP, std::string("patch fields: ") + hipGetErrorString(e));
   return LBM_OK;
