@@ -488,9 +488,35 @@ int lbm_get_populations(lbm_ctx* c, double* f) {
 
 }  // extern "C"
 
-int lbm_enqueue_step_from(lbm_ctx* c, const void* src, void* dst) {
+namespace {
+// whether two steps may go in one launch; the coupling re-collides its cells between two steps
+bool pairs(const lbm_ctx* c) {
+  return !(c->couple_on && c->ncouple) && lbm::pair_fits(c->g, c->esize, c->walls);
+}
+
+int step_from(lbm_ctx* c, const void* src, void* dst) {
   HIPCHK(c, lbm::launch_dense_step(c->g, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls,
                                    c->p64, c->p32, lbm::BoundaryArgs{c->d_bct, c->d_bcu}, c->spec, c->stream));
+  return LBM_OK;
+}
+
+int pair_from(lbm_ctx* c, const void* src, void* dst) {
+  HIPCHK(c, lbm::launch_dense_pair(c->g, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls, c->p64,
+                                   c->p32, lbm::BoundaryArgs{c->d_bct, c->d_bcu}, c->stream));
+  return LBM_OK;
+}
+}  // namespace
+
+int lbm_enqueue_run(lbm_ctx* c, const void* src, int nsteps, void* dst, const void** out) {
+  const bool two = pairs(c);
+  for (int k; nsteps > 0; nsteps -= k) {
+    k = two && nsteps >= 2 ? 2 : 1;
+    void* d = dst && nsteps == k ? dst : c->buf[src == c->buf[0] ? 1 : 0];
+    const int rc = k == 2 ? pair_from(c, src, d) : step_from(c, src, d);
+    if (rc) return rc;
+    src = d;
+  }
+  if (out) *out = src;
   return LBM_OK;
 }
 
@@ -508,20 +534,16 @@ int lbm_enqueue_steps(lbm_ctx* c, int nsteps, bool single) {
     return LBM_OK;
   }
   int s = 0;
-  // the coupling re-collides its cells between two steps
-  if (!single && !(c->couple_on && c->ncouple) && lbm::pair_fits(c->g, c->esize, c->walls)) {
+  if (!single && pairs(c)) {
     for (; s + 2 <= nsteps; s += 2) {
-      HIPCHK(c, lbm::launch_dense_pair(c->g, c->fp32, c->f32math, c->buf[c->cur], c->buf[c->cur ^ 1], c->words, c->alpha,
-                                       c->force, c->walls, c->p64, c->p32, lbm::BoundaryArgs{c->d_bct, c->d_bcu},
-                                       c->stream));
+      const int rc = pair_from(c, c->buf[c->cur], c->buf[c->cur ^ 1]);
+      if (rc) return rc;
       c->cur ^= 1;
     }
   }
   for (; s < nsteps; s++) {
-    HIPCHK(c, lbm::launch_dense_step(c->g, c->fp32, c->f32math, c->buf[c->cur], c->buf[c->cur ^ 1], c->words,
-                                     c->alpha, c->force, c->walls, c->p64, c->p32,
-                                     lbm::BoundaryArgs{c->d_bct, c->d_bcu}, c->spec, c->stream));
-    const int rc = lbm_enqueue_coupling(c, c->buf[c->cur], c->buf[c->cur ^ 1]);
+    int rc = step_from(c, c->buf[c->cur], c->buf[c->cur ^ 1]);
+    if (!rc) rc = lbm_enqueue_coupling(c, c->buf[c->cur], c->buf[c->cur ^ 1]);
     if (rc) return rc;
     c->cur ^= 1;
   }

@@ -86,8 +86,10 @@ inline lbm::DenseGeom lbm_state_geom(const lbm_ctx* c) {
   g.layout = !c->aa ? lbm::LAYOUT_PULL : (c->parity ? lbm::LAYOUT_AA_SWAPPED : lbm::LAYOUT_AA_NATURAL);
   return g;
 }
-// one step from src into dst (any two state-sized device buffers), leaving buf/cur alone
-int lbm_enqueue_step_from(lbm_ctx* c, const void* src, void* dst);
+// nsteps steps from the state in src (two-buffer layout, no coupling), the last one written to dst (neither
+// of the context's buffers, or null: to one of them); the states in between go through the context's
+// buffers, cur stays.  *out = where the result lies.
+int lbm_enqueue_run(lbm_ctx* c, const void* src, int nsteps, void* dst, const void** out);
 // re-collision of the MD-coupled cells for the step src -> dst (no-op without coupling)
 int lbm_enqueue_coupling(lbm_ctx* c, const void* src, void* dst);
 // in-place layout: save the coupled cells' populations before a step, re-collide them after it
