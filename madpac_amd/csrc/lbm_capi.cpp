@@ -490,8 +490,11 @@ int lbm_get_populations(lbm_ctx* c, double* f) {
 
 namespace {
 // whether two steps may go in one launch; the coupling re-collides its cells between two steps
-bool pairs(const lbm_ctx* c) {
-  return !(c->couple_on && c->ncouple) && lbm::pair_fits(c->g, c->esize, c->walls);
+bool pairs(const lbm_ctx* c, lbm::PairGeom* plan) {
+  if (c->couple_on && c->ncouple) return false;
+  bool open = false;
+  for (const lbm::BoundaryClass& b : c->bct) open = open || (b.mask && (b.type & lbm::BC_TYPE_MASK) != lbm::BC_MOVING_WALL);
+  return lbm::pair_plan(c->g, c->esize, c->force || c->alpha || c->walls, open, plan);
 }
 
 int step_from(lbm_ctx* c, const void* src, void* dst) {
@@ -500,19 +503,20 @@ int step_from(lbm_ctx* c, const void* src, void* dst) {
   return LBM_OK;
 }
 
-int pair_from(lbm_ctx* c, const void* src, void* dst) {
-  HIPCHK(c, lbm::launch_dense_pair(c->g, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls, c->p64,
+int pair_from(lbm_ctx* c, const lbm::PairGeom& plan, const void* src, void* dst) {
+  HIPCHK(c, lbm::launch_dense_pair(c->g, plan, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls, c->p64,
                                    c->p32, lbm::BoundaryArgs{c->d_bct, c->d_bcu}, c->stream));
   return LBM_OK;
 }
 }  // namespace
 
 int lbm_enqueue_run(lbm_ctx* c, const void* src, int nsteps, void* dst, const void** out) {
-  const bool two = pairs(c);
+  lbm::PairGeom plan;
+  const bool two = nsteps >= 2 && pairs(c, &plan);
   for (int k; nsteps > 0; nsteps -= k) {
     k = two && nsteps >= 2 ? 2 : 1;
     void* d = dst && nsteps == k ? dst : c->buf[src == c->buf[0] ? 1 : 0];
-    const int rc = k == 2 ? pair_from(c, src, d) : step_from(c, src, d);
+    const int rc = k == 2 ? pair_from(c, plan, src, d) : step_from(c, src, d);
     if (rc) return rc;
     src = d;
   }
@@ -534,9 +538,10 @@ int lbm_enqueue_steps(lbm_ctx* c, int nsteps, bool single) {
     return LBM_OK;
   }
   int s = 0;
-  if (!single && pairs(c)) {
+  lbm::PairGeom plan;
+  if (!single && nsteps >= 2 && pairs(c, &plan)) {
     for (; s + 2 <= nsteps; s += 2) {
-      const int rc = pair_from(c, c->buf[c->cur], c->buf[c->cur ^ 1]);
+      const int rc = pair_from(c, plan, c->buf[c->cur], c->buf[c->cur ^ 1]);
       if (rc) return rc;
       c->cur ^= 1;
     }

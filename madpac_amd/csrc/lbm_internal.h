@@ -131,10 +131,12 @@ struct PairGeom {
   int tx, ty, tz;  // tiles of columns along x and y, chunks along z
   int cz;          // planes per chunk
   int64_t nblocks, nblocks_padded;
+  int64_t passes;  // planes that one CU sweeps in sequence, pipeline fill included
 };
-// whether launch_dense_pair takes this lattice and is the faster way
-bool pair_fits(const DenseGeom& g, size_t esize, bool walls);
-hipError_t launch_dense_pair(const DenseGeom& g, bool fp32, bool f32math, const void* src, void* dst,
+// The split of this lattice, and whether launch_dense_pair takes it and is the faster way.
+// extra: force, porosity or boundary classes; open: classes other than moving walls.
+bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, PairGeom* plan);
+hipError_t launch_dense_pair(const DenseGeom& g, const PairGeom& plan, bool fp32, bool f32math, const void* src, void* dst,
                              const uint32_t* words, const void* alpha, bool force, bool walls, const CollideParams& p64,
                              const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t stream);
 // reference state f (FP64) from the stored state

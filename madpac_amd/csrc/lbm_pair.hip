@@ -67,11 +67,19 @@ __global__ __launch_bounds__((Tile<TX, TY>::THREADS), 3) void k_dense_pair(
     const T* __restrict__ alpha, CollideParams p64, CollideParams32 p32, BoundaryArgs bc) {
   using Sh = Tile<TX, TY>;
   __shared__ T lds[2 * SLOTS * Sh::STRIDE];
+  // the boundary classes, kept near: from global memory, a classed cell's mask and target were two more
+  // round trips in each of a plane's two collisions (channel 131 x 70 x 53 FP64 37.7 -> 36.4 us a step)
+  __shared__ BoundaryClass classes[WALLS ? MAX_CLASSES : 1];
   const int tid = (int)threadIdx.x;
   // XCD-contiguous ranges of tiles (x fastest, then y, then the z chunks)
   const int64_t bid = blockIdx.x;
   const int64_t b = (bid % NXCD) * (pg.nblocks_padded / NXCD) + bid / NXCD;
   if (b >= pg.nblocks) return;
+  if constexpr (WALLS) {
+    if (tid < MAX_CLASSES) classes[tid] = bc.table[tid];
+    __syncthreads();
+    bc.table = classes;
+  }
   const int tx = (int)(b % pg.tx), ty = (int)((b / pg.tx) % pg.ty), tz = (int)(b / ((int64_t)pg.tx * pg.ty));
   const int x0 = tx * TX, y0 = ty * TY, z0 = tz * pg.cz, z1 = min(g.nz, z0 + pg.cz);
   const int vx = min(TX, g.nx - x0), vy = min(TY, g.ny - y0);
@@ -269,18 +277,19 @@ __global__ __launch_bounds__((Tile<TX, TY>::THREADS), 3) void k_dense_pair(
 // 24), 64^3 32 chunks of 2 (13.2 us; 16.2 in 16 chunks).
 constexpr int NCU = 256;
 
-template <int TX, int TY>
-PairGeom pair_geom(const DenseGeom& g) {
+PairGeom pair_geom(const DenseGeom& g, int tile_x, int tile_y) {
   PairGeom p;
-  p.tx = (g.nx + TX - 1) / TX;
-  p.ty = (g.ny + TY - 1) / TY;
+  p.tx = (g.nx + tile_x - 1) / tile_x;
+  p.ty = (g.ny + tile_y - 1) / tile_y;
   const int64_t tiles = (int64_t)p.tx * p.ty;
-  int64_t best = INT64_MAX;
-  for (int n = 1; n <= g.nz; n++) {
+  p.passes = INT64_MAX;
+  // (beyond eight rounds, shorter chunks only add planes computed twice)
+  const int64_t most = std::min<int64_t>(g.nz, 8 * NCU / std::min<int64_t>(tiles, NCU));
+  for (int n = 1; n <= most; n++) {
     const int cz = (g.nz + n - 1) / n;
     const int64_t rounds = (tiles * ((g.nz + cz - 1) / cz) + NCU - 1) / NCU, cost = rounds * (cz + 3);
-    if (cost < best) {
-      best = cost;
+    if (cost < p.passes) {
+      p.passes = cost;
       p.cz = cz;
     }
   }
@@ -291,9 +300,8 @@ PairGeom pair_geom(const DenseGeom& g) {
 }
 
 template <typename T, bool M32, bool AOS, int TX, int TY>
-hipError_t pair_t(const DenseGeom& g, const void* src, void* dst, const uint32_t* words, const void* alpha, bool force,
+hipError_t pair_t(const DenseGeom& g, const PairGeom& pg, const void* src, void* dst, const uint32_t* words, const void* alpha, bool force,
                   bool walls, const CollideParams& p64, const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t s) {
-  const PairGeom pg = pair_geom<TX, TY>(g);
   const dim3 grid((unsigned)pg.nblocks_padded), block(Tile<TX, TY>::THREADS);
 #define LBM_PAIR(F, A, W)                                                                                        \
   hipLaunchKernelGGL((k_dense_pair<T, F, A, W, M32, AOS, TX, TY>), grid, block, 0, s, g, pg, (const T*)src, (T*)dst, \
@@ -314,45 +322,60 @@ hipError_t pair_t(const DenseGeom& g, const void* src, void* dst, const uint32_t
 }
 
 template <typename T, bool M32, bool AOS>
-hipError_t pair_tile(const DenseGeom& g, const void* src, void* dst, const uint32_t* words, const void* alpha, bool force,
+hipError_t pair_tile(const DenseGeom& g, const PairGeom& pg, const void* src, void* dst, const uint32_t* words, const void* alpha, bool force,
                      bool walls, const CollideParams& p64, const CollideParams32& p32, const BoundaryArgs& bc,
                      hipStream_t s) {
   if constexpr (sizeof(T) == 8) {
     if (g.bricked)
-      return pair_t<T, M32, AOS, 32, 16>(g, src, dst, words, alpha, force, walls, p64, p32, bc, s);
+      return pair_t<T, M32, AOS, 32, 16>(g, pg, src, dst, words, alpha, force, walls, p64, p32, bc, s);
   }
-  return pair_t<T, M32, AOS, 64, 8>(g, src, dst, words, alpha, force, walls, p64, p32, bc, s);
+  return pair_t<T, M32, AOS, 64, 8>(g, pg, src, dst, words, alpha, force, walls, p64, p32, bc, s);
 }
 
 template <bool AOS>
-hipError_t pair_type(const DenseGeom& g, bool fp32, bool f32math, const void* src, void* dst, const uint32_t* words,
+hipError_t pair_type(const DenseGeom& g, const PairGeom& pg, bool fp32, bool f32math, const void* src, void* dst, const uint32_t* words,
                      const void* alpha, bool force, bool walls, const CollideParams& p64, const CollideParams32& p32,
                      const BoundaryArgs& bc, hipStream_t s) {
   if (fp32 && f32math)
-    return pair_tile<float, true, AOS>(g, src, dst, words, alpha, force, walls, p64, p32, bc, s);
-  if (fp32) return pair_tile<float, false, AOS>(g, src, dst, words, alpha, force, walls, p64, p32, bc, s);
-  return pair_tile<double, false, AOS>(g, src, dst, words, alpha, force, walls, p64, p32, bc, s);
+    return pair_tile<float, true, AOS>(g, pg, src, dst, words, alpha, force, walls, p64, p32, bc, s);
+  if (fp32) return pair_tile<float, false, AOS>(g, pg, src, dst, words, alpha, force, walls, p64, p32, bc, s);
+  return pair_tile<double, false, AOS>(g, pg, src, dst, words, alpha, force, walls, p64, p32, bc, s);
 }
 
 }  // namespace
 
-// The smallest lattices stay with the one-step kernel: a sweep takes four planes' time at least, 4-5 us
-// each on one CU, and cells with boundary classes make its waves longer.  Measured per step, one-step
-// against this kernel: FP64 64 x 64 x 48 periodic 13.4 / 11.8 us, cavity 14.1 / 14.1; 64^3 16.4 / 13.2,
-// cavity 17.2 / 15.0, channel 16.2 / 19.3; 131 x 70 x 53 periodic 39.9 / 26.6, cavity 41.3 / 28.0, channel
-// 41.2 / 37.5; FP32 64^3 9.7 / 9.0, cavity 10.0 / 11.4; 131 x 70 x 53 25.0 / 18.2, cavity 25.1 / 21.0.
+// The rule weighs two launches of the one-step kernel against one of this kernel, in microseconds.
+//  * One step: 3 and its bytes at 5.3 TB/s, with half of the lanes that rows leave idle, and a fifth more
+//    where rows do not start on 128-byte lines.
+//  * This kernel: its planes in sequence (PairGeom::passes), each a latency: loads, two collisions, two
+//    barriers.  Force, porosity and boundary classes lengthen the collisions, open boundaries most: their
+//    cells' two equilibria per link hold up the whole workgroup.
+// Measured per step, one-step / this kernel (FP32 96^3 periodic 30.9 / 31.4, force and porosity 30.7 / 37.8, lid
+// 31.8 / 36.8, channel 35.2 / 48.4; 128^3 55.3 / 46.7, force and porosity 56.6 / 54.2; 192^3 187 / 167,
+// channel 189 / 240; 256^3 458 / 355, channel 502 / 530.  FP64 64^3 16.8 / 12.8, force and porosity 17.0 / 15.3,
+// lid 17.2 / 15.0, channel 16.2 / 19.3; 80^3 36.3 / 26.1, channel 38.1 / 39.1; 131 x 70 x 53 40.2 / 27.0,
+// channel 41.4 / 36.4; 256^3 932 / 527).  The microseconds of a plane are this table's.
 // A plane of populations has to fit the 32-bit offsets.
-bool pair_fits(const DenseGeom& g, size_t esize, bool walls) {
+bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, PairGeom* plan) {
   const int64_t plane = g.bricked ? (int64_t)64 * g.bnx * g.bny : (int64_t)g.nx * g.ny;
-  return g.Nu >= (walls ? (int64_t)3 << 17 : (int64_t)1 << 18) &&
-         plane * (g.aos ? Q : 1) * (int64_t)esize <= (int64_t)UINT32_MAX;
+  if (plane * (g.aos ? Q : 1) * (int64_t)esize > (int64_t)UINT32_MAX) return false;
+  const bool f64 = esize == 8;
+  *plan = f64 && g.bricked ? pair_geom(g, 32, 16) : pair_geom(g, 64, 8);
+  double cells = (double)g.Nu;
+  if (!g.bricked) {
+    cells *= 0.5 + 0.5 * ((g.nx + 63) / 64 * 64) / g.nx;
+    if ((g.nx * esize) % 128) cells *= 1.2;
+  }
+  const double step = 3.0 + cells * 2 * Q * (double)esize / 5.3e6;
+  const double pass = open ? 8.5 : f64 ? (extra ? 7.0 : 6.0) : (extra ? 5.7 : 5.1);
+  return (double)plan->passes * pass < 2.0 * step;
 }
 
-hipError_t launch_dense_pair(const DenseGeom& g, bool fp32, bool f32math, const void* src, void* dst,
+hipError_t launch_dense_pair(const DenseGeom& g, const PairGeom& pg, bool fp32, bool f32math, const void* src, void* dst,
                              const uint32_t* words, const void* alpha, bool force, bool walls, const CollideParams& p64,
                              const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t s) {
-  return g.aos ? pair_type<true>(g, fp32, f32math, src, dst, words, alpha, force, walls, p64, p32, bc, s)
-               : pair_type<false>(g, fp32, f32math, src, dst, words, alpha, force, walls, p64, p32, bc, s);
+  return g.aos ? pair_type<true>(g, pg, fp32, f32math, src, dst, words, alpha, force, walls, p64, p32, bc, s)
+               : pair_type<false>(g, pg, fp32, f32math, src, dst, words, alpha, force, walls, p64, p32, bc, s);
 }
 
 }  // namespace lbm

@@ -69,3 +69,17 @@ def test_pairs_in_a_captured_graph():
                 lat.step(n, graph=graph)
             out.append(lat.get_populations())
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("size, scene, prec, order", [
+    ((127, 100, 90), "cavity", lbm.FP32_SHIFTED, ROWS),       # planes, one idle lane, last tile of four rows
+    ((191, 97, 90), "open", lbm.FP32_SHIFTED, ROWS),          # last tile of one row
+    ((130, 120, 118), "brinkman", lbm.FP32_SHIFTED, ROWS),    # last tile of two columns
+    ((127, 125, 121), "porous", lbm.FP32_SHIFTED, BRICKS),    # bricks cut by the box
+    ((128, 130, 120), "porous", lbm.FP32_SHIFTED_F32, ROWS),  # interleaved rows
+    ((97, 90, 93), "cavity", lbm.FP64, BRICKS),               # boundary classes in bricks
+    ((98, 90, 88), "channel", lbm.FP64, ROWS),                # inlet and outlet classes of a parabolic profile
+])
+def test_pairs_equal_single_steps_where_they_pay(size, scene, prec, order):
+    # sizes that the rule of pair_plan sends to the two-step kernel, with each kind of boundary it weighs
+    test_pairs_equal_single_steps(size, scene, prec, order)
