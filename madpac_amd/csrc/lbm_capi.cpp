@@ -489,34 +489,48 @@ int lbm_get_populations(lbm_ctx* c, double* f) {
 }  // extern "C"
 
 namespace {
-// whether two steps may go in one launch; the coupling re-collides its cells between two steps
-bool pairs(const lbm_ctx* c, lbm::PairGeom* plan) {
-  if (c->couple_on && c->ncouple) return false;
+// How a run of steps is cut into launches: up to `most` steps in each, by the kernel for small lattices or
+// by the two-step kernel.
+struct StepPlan {
+  int most = 1;
+  bool small = false;
+  lbm::PairGeom pair;
+};
+
+StepPlan plan_steps(const lbm_ctx* c) {
+  StepPlan p;
+  if (c->couple_on && c->ncouple) return p;  // the coupling re-collides its cells between two steps
+  p.most = lbm::small_steps(c->g);
+  p.small = p.most > 1;
+  if (p.small) return p;
   bool open = false;
   for (const lbm::BoundaryClass& b : c->bct) open = open || (b.mask && (b.type & lbm::BC_TYPE_MASK) != lbm::BC_MOVING_WALL);
-  return lbm::pair_plan(c->g, c->esize, c->force || c->alpha || c->walls, open, plan);
+  if (lbm::pair_plan(c->g, c->esize, c->force || c->alpha || c->walls, open, &p.pair)) p.most = 2;
+  return p;
 }
 
-int step_from(lbm_ctx* c, const void* src, void* dst) {
-  HIPCHK(c, lbm::launch_dense_step(c->g, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls,
-                                   c->p64, c->p32, lbm::BoundaryArgs{c->d_bct, c->d_bcu}, c->spec, c->stream));
-  return LBM_OK;
-}
-
-int pair_from(lbm_ctx* c, const lbm::PairGeom& plan, const void* src, void* dst) {
-  HIPCHK(c, lbm::launch_dense_pair(c->g, plan, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls, c->p64,
-                                   c->p32, lbm::BoundaryArgs{c->d_bct, c->d_bcu}, c->stream));
+// k <= p.most steps src -> dst
+int launch_steps(lbm_ctx* c, const StepPlan& p, int k, const void* src, void* dst) {
+  const lbm::BoundaryArgs bc{c->d_bct, c->d_bcu};
+  if (k == 1)
+    HIPCHK(c, lbm::launch_dense_step(c->g, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls, c->p64,
+                                     c->p32, bc, c->spec, c->stream));
+  else if (p.small)
+    HIPCHK(c, lbm::launch_dense_small(c->g, k, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls,
+                                      c->p64, c->p32, bc, c->stream));
+  else
+    HIPCHK(c, lbm::launch_dense_pair(c->g, p.pair, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls,
+                                     c->p64, c->p32, bc, c->stream));
   return LBM_OK;
 }
 }  // namespace
 
 int lbm_enqueue_run(lbm_ctx* c, const void* src, int nsteps, void* dst, const void** out) {
-  lbm::PairGeom plan;
-  const bool two = nsteps >= 2 && pairs(c, &plan);
+  const StepPlan p = plan_steps(c);
   for (int k; nsteps > 0; nsteps -= k) {
-    k = two && nsteps >= 2 ? 2 : 1;
+    k = std::min(nsteps, p.most);
     void* d = dst && nsteps == k ? dst : c->buf[src == c->buf[0] ? 1 : 0];
-    const int rc = k == 2 ? pair_from(c, plan, src, d) : step_from(c, src, d);
+    const int rc = launch_steps(c, p, k, src, d);
     if (rc) return rc;
     src = d;
   }
@@ -537,17 +551,10 @@ int lbm_enqueue_steps(lbm_ctx* c, int nsteps, bool single) {
     }
     return LBM_OK;
   }
-  int s = 0;
-  lbm::PairGeom plan;
-  if (!single && nsteps >= 2 && pairs(c, &plan)) {
-    for (; s + 2 <= nsteps; s += 2) {
-      const int rc = pair_from(c, plan, c->buf[c->cur], c->buf[c->cur ^ 1]);
-      if (rc) return rc;
-      c->cur ^= 1;
-    }
-  }
-  for (; s < nsteps; s++) {
-    int rc = step_from(c, c->buf[c->cur], c->buf[c->cur ^ 1]);
+  const StepPlan p = single || nsteps < 2 ? StepPlan{} : plan_steps(c);
+  for (int k; nsteps > 0; nsteps -= k) {
+    k = std::min(nsteps, p.most);
+    int rc = launch_steps(c, p, k, c->buf[c->cur], c->buf[c->cur ^ 1]);
     if (!rc) rc = lbm_enqueue_coupling(c, c->buf[c->cur], c->buf[c->cur ^ 1]);
     if (rc) return rc;
     c->cur ^= 1;
@@ -617,13 +624,14 @@ int lbm_step_graph(lbm_ctx* c, int nsteps) {
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->cfg.device));
   const int slot = c->aa ? c->parity : c->cur;
-  const int K = GRAPH_STEPS;
+  // an even number of launches, so that cur (or parity) ends at this slot's phase
+  const int most = c->aa ? 1 : plan_steps(c).most, K = most > 2 ? 12 * most : GRAPH_STEPS;
   if (nsteps >= K) {
     const lbm_graph_key key = graph_key(c);
     if (!c->gexec[slot] || !(c->gkey[slot] == key)) {
       graph_release(c, slot);
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      rc = lbm_enqueue_steps(c, K);  // K even: cur (or parity) ends at this slot's phase
+      rc = lbm_enqueue_steps(c, K);
       hipGraph_t g = nullptr;
       const hipError_t e = hipStreamEndCapture(c->stream, &g);
       if (rc) {

@@ -139,6 +139,13 @@ bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, PairGeom
 hipError_t launch_dense_pair(const DenseGeom& g, const PairGeom& plan, bool fp32, bool f32math, const void* src, void* dst,
                              const uint32_t* words, const void* alpha, bool force, bool walls, const CollideParams& p64,
                              const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t stream);
+// How many steps launch_dense_small takes at once on this lattice; 1 where other kernels are faster.
+int small_steps(const DenseGeom& g);
+// `steps` (2 to small_steps) steps src -> dst in one launch on a small lattice (lbm_small.hip): the same state
+// as single steps
+hipError_t launch_dense_small(const DenseGeom& g, int steps, bool fp32, bool f32math, const void* src, void* dst,
+                              const uint32_t* words, const void* alpha, bool force, bool walls, const CollideParams& p64,
+                              const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t stream);
 // reference state f (FP64) from the stored state
 // one in-place AA step on a single buffer: parity 0 reads the NATURAL layout and leaves SWAPPED,
 // parity 1 the reverse
