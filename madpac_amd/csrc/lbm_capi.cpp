@@ -102,8 +102,9 @@ int switch_cell_order(lbm_ctx* c, bool bricks) {
                              c->stream));
   }
   if (c->ncouple) HIPCHK(c, lbm::launch_convert_ids(from, to, c->d_ccells, c->ncouple, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   c->g = to;
+  if (c->ncouple) HIPCHK(c, lbm_couple_index(c));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   return LBM_OK;
 }
 
@@ -494,18 +495,20 @@ namespace {
 struct StepPlan {
   int most = 1;
   bool small = false;
+  bool coupled = false;  // two steps, then those of the boxes around the coupled cells again with the coupling
   lbm::PairGeom pair;
 };
 
 StepPlan plan_steps(const lbm_ctx* c) {
   StepPlan p;
-  if (c->couple_on && c->ncouple) return p;  // the coupling re-collides its cells between two steps
-  p.most = lbm::small_steps(c->g);
+  p.coupled = c->couple_on && c->ncouple;
+  if (p.coupled && (!c->ncboxes || c->force || c->alpha)) return p;  // single steps, each with its re-collision
+  if (!p.coupled) p.most = lbm::small_steps(c->g);
   p.small = p.most > 1;
   if (p.small) return p;
   bool open = false;
   for (const lbm::BoundaryClass& b : c->bct) open = open || (b.mask && (b.type & lbm::BC_TYPE_MASK) != lbm::BC_MOVING_WALL);
-  if (lbm::pair_plan(c->g, c->esize, c->force || c->alpha || c->walls, open, &p.pair)) p.most = 2;
+  if (lbm::pair_plan(c->g, c->esize, c->force || c->alpha || c->walls, open, p.coupled ? c->ncboxes : 0, &p.pair)) p.most = 2;
   return p;
 }
 
@@ -518,9 +521,13 @@ int launch_steps(lbm_ctx* c, const StepPlan& p, int k, const void* src, void* ds
   else if (p.small)
     HIPCHK(c, lbm::launch_dense_small(c->g, k, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls,
                                       c->p64, c->p32, bc, c->stream));
-  else
+  else {
     HIPCHK(c, lbm::launch_dense_pair(c->g, p.pair, c->fp32, c->f32math, src, dst, c->words, c->alpha, c->force, c->walls,
                                      c->p64, c->p32, bc, c->stream));
+    if (p.coupled)
+      HIPCHK(c, lbm::launch_coupled_boxes(c->g, c->fp32, c->f32math, src, dst, c->words, c->walls, c->p64, c->p32, bc,
+                                          lbm_couple_args(c), c->d_cidx, c->d_cboxes, c->ncboxes, c->stream));
+  }
   return LBM_OK;
 }
 }  // namespace
@@ -555,7 +562,7 @@ int lbm_enqueue_steps(lbm_ctx* c, int nsteps, bool single) {
   for (int k; nsteps > 0; nsteps -= k) {
     k = std::min(nsteps, p.most);
     int rc = launch_steps(c, p, k, c->buf[c->cur], c->buf[c->cur ^ 1]);
-    if (!rc) rc = lbm_enqueue_coupling(c, c->buf[c->cur], c->buf[c->cur ^ 1]);
+    if (!rc && k == 1) rc = lbm_enqueue_coupling(c, c->buf[c->cur], c->buf[c->cur ^ 1]);
     if (rc) return rc;
     c->cur ^= 1;
   }

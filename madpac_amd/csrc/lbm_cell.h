@@ -93,6 +93,8 @@ __device__ __forceinline__ double cdot64(int q, double v0, double v1, double v2)
 __device__ __forceinline__ double over_cs2(double x) { return __builtin_fma(3.0, x, x * 0x1.8p-53); }
 __device__ __forceinline__ double over_cs2x2(double x) { return __builtin_fma(1.5, x, x * 0x1.8p-54); }
 __device__ __forceinline__ double over_cs4x2(double x) { return __builtin_fma(4.5, x, x * 0x1.2p-52); }
+// (1.0/3.0)*(1.0/3.0) of the coupling's force term is half of the third constant: the same proof, z = 9
+__device__ __forceinline__ double over_cs4(double x) { return __builtin_fma(9.0, x, x * 0x1.2p-51); }
 
 // computeFeq (BLB/BlockComputeCellValues.cpp:14-20) of direction q (cu = c_q . u, du = u.u / (2 cs2))
 // and of its mirror 18 - q, whose c . u is -cu and whose weight is the same: cu / cs2 changes its sign

@@ -11,113 +11,26 @@
 // from populations saved before the step); the hot kernel is unchanged.  A gather kernel returns rho
 // and u of the coupled cells as getAndSetV exports them (after its GET block).  Coupled cells use the reference's block-solver
 // collision: no body force and no porosity (the host rejects those combinations).
+#include <algorithm>
 #include <cmath>
 #include <string>
 #include <vector>
 
+#include "lbm_couple.h"
 #include "lbm_ctx.h"
 #include "lbm_geom.h"
 
 namespace lbm {
 
-struct CoupleArgs {
-  const int64_t* cells;   // coupled cell indices
-  int64_t n;
-  const double* u;        // [3n] MD velocity (lattice units)
-  const double* rho;      // [n] MD density or null
-  int mode;               // LBM_COUPLE_*
-  double dt;              // LB time step of the Dirichlet forcing
-  double tau;             // configured tau (computeGi's _tau)
-  double omega;           // 1 / tau_eff (BlockBGK)
-};
-
-
-// The GET block of getAndSetV (:100-129) for coupled cell k, on the cell's rho and u: overwrite sets
-// u = u_MD (:121-122); Dirichlet computes g = (u_MD - u)/dt and shifts u += dt/2 g (:110-117); with
-// density coupling rho = rho_MD (:124-129).  g stays 0 in the overwrite mode.
-__device__ __forceinline__ void couple_get(const CoupleArgs& a, int64_t k, double& rho, double (&u)[3],
-                                           double (&g)[3]) {
-  const double* um = a.u + 3 * k;
-  g[0] = g[1] = g[2] = 0.0;
-  if (a.mode == LBM_COUPLE_DIRICHLET) {
-    for (int d = 0; d < 3; d++) {
-      g[d] = (um[d] - u[d]) / a.dt;
-      u[d] += a.dt / 2.0 * g[d];
-    }
-  } else {
-    for (int d = 0; d < 3; d++) u[d] = um[d];
-  }
-  if (a.rho) rho = a.rho[k];
+// k of the coupled cells, -1 of the others (one entry per stored cell), for the boxes of lbm_small.hip.
+__global__ __launch_bounds__(256) void k_couple_clear(int32_t* __restrict__ idx, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) idx[i] = -1;
 }
-
-// FP64 collision of one coupled cell (reference operation order, as the oracle restates it).
-__device__ __forceinline__ double collide_coupled_f64(double (&f)[Q], const CoupleArgs& a, int64_t k,
-                                                      double (&uo)[3]) {
-  double rho = 0.0;
-#pragma unroll
-  for (int q = 0; q < Q; q++) rho += f[q];
-  double b0 = 0.0, b1 = 0.0, b2 = 0.0;
-#pragma unroll
-  for (int q = 0; q < Q; q++) {
-    if (CX(q) == 1) b0 += f[q];
-    if (CX(q) == -1) b0 -= f[q];
-    if (CY(q) == 1) b1 += f[q];
-    if (CY(q) == -1) b1 -= f[q];
-    if (CZ(q) == 1) b2 += f[q];
-    if (CZ(q) == -1) b2 -= f[q];
-  }
-  const double inv = 1.0 / rho;
-  double u[3] = {b0 * inv, b1 * inv, b2 * inv};
-  double g[3];
-  couple_get(a, k, rho, u, g);
-  const bool dir = a.mode == LBM_COUPLE_DIRICHLET;
-  uo[0] = u[0];
-  uo[1] = u[1];
-  uo[2] = u[2];
-  double uu = u[0] * u[0];
-  uu += u[1] * u[1];
-  uu += u[2] * u[2];
-  const double du = over_cs2x2(uu);
-  f[REST] -= a.omega * (f[REST] - W64(REST) * rho * (1.0 - du));
-#pragma unroll
-  for (int q = 0; q < REST; q++) {
-    const FeqPair e = feq_pair_f64(q, rho, cdot64(q, u[0], u[1], u[2]), du);
-    f[q] -= a.omega * (f[q] - e.q);
-    f[Q - 1 - q] -= a.omega * (f[Q - 1 - q] - e.mirror);
-  }
-  if (dir) {
-    // adjustF / computeGi, with (c.u)^2 as the reference writes it
-    const double pref = 1.0 - 0.5 / a.tau;
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-      const double m0 = (double)CX(q) - u[0], m1 = (double)CY(q) - u[1], m2 = (double)CZ(q) - u[2];
-      double cmg = m0 * g[0];
-      cmg += m1 * g[1];
-      cmg += m2 * g[2];
-      const double cu = cdot64(q, u[0], u[1], u[2]);
-      const double cg = cdot64(q, g[0], g[1], g[2]);
-      const double gi = pref * W64(q) * rho *
-                        (1.0 / (1.0 / 3.0) * cmg + (cu * cu) / ((1.0 / 3.0) * (1.0 / 3.0)) * cg);
-      f[q] += a.dt * gi;
-    }
-  }
-  return rho;
-}
-
-// Coupled collision of cell k (stored index i, flag word w), then the boundary class of its links.
-template <bool WALLS>
-__device__ __forceinline__ void couple_collide(double (&f)[Q], const CoupleArgs& a, int64_t k, int64_t i, uint32_t w,
-                                               const BoundaryArgs& bc) {
-  double u[3];
-  const double rho = collide_coupled_f64(f, a, k, u);
-  if (WALLS) {
-    const uint32_t cls = (w >> CLASS_SHIFT) & CLASS_BITS;
-    if (cls) {
-      const BoundaryClass& b = bc.table[cls];
-      const uint32_t m = w & b.mask;
-      if (m) apply_boundary_f64(f, m, b, bc.cell_u, i, rho, u[0], u[1], u[2]);
-    }
-  }
+__global__ __launch_bounds__(256) void k_couple_index(const int64_t* __restrict__ cells, int64_t n,
+                                                      int32_t* __restrict__ idx) {
+  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (k < n) idx[cells[k]] = (int32_t)k;
 }
 
 // Re-collide the coupled cells from src and overwrite their own output slots in dst (run after the
@@ -131,15 +44,12 @@ __global__ __launch_bounds__(256) void k_couple(DenseGeom g, const T* __restrict
   const uint32_t w = words[i];
   if (!(w & FLUID)) return;
   const NbrOff o = nbr_offsets(g, pos_of(g, i));
-  double f[Q];
+  T f[Q];
 #pragma unroll
-  for (int q = 0; q < Q; q++) {
-    const T v = src[pull_index(g, q, w, i, o)];
-    f[q] = sizeof(T) == 8 ? (double)v : (double)v + W64(q);
-  }
-  couple_collide<WALLS>(f, a, k, i, w, bc);
+  for (int q = 0; q < Q; q++) f[q] = src[pull_index(g, q, w, i, o)];
+  couple_cell<T, WALLS>(f, a, k, i, w, bc);
 #pragma unroll
-  for (int q = 0; q < Q; q++) dst[pop_at(g, q, i)] = sizeof(T) == 8 ? (T)f[q] : (T)(f[q] - W64(q));
+  for (int q = 0; q < Q; q++) dst[pop_at(g, q, i)] = f[q];
 }
 
 // In-place (AA) layout: the step overwrites the populations the re-collision starts from, so they
@@ -241,11 +151,23 @@ int cfail(lbm_ctx* c, int code, const std::string& msg) {
 }
 }  // namespace
 
+lbm::CoupleArgs lbm_couple_args(const lbm_ctx* c) {
+  return lbm::CoupleArgs{c->d_ccells, c->ncouple, c->d_cu, c->couple_rho ? c->d_crho : nullptr, c->couple_mode,
+                         c->couple_dt, c->cfg.tau, c->p64.omega};
+}
+
+hipError_t lbm_couple_index(lbm_ctx* c) {
+  if (!c->d_cidx) return hipSuccess;
+  hipLaunchKernelGGL(lbm::k_couple_clear, dim3((unsigned)((c->g.N + 255) / 256)), dim3(256), 0, c->stream, c->d_cidx, c->g.N);
+  hipLaunchKernelGGL(lbm::k_couple_index, dim3((unsigned)((c->ncouple + 255) / 256)), dim3(256), 0, c->stream,
+                     c->d_ccells, c->ncouple, c->d_cidx);
+  return hipGetLastError();
+}
+
 // Launch the re-collision of the coupled cells for the step src -> dst (called by the step loop).
 int lbm_enqueue_coupling(lbm_ctx* c, const void* src, void* dst) {
   if (!c->couple_on || c->ncouple == 0) return LBM_OK;
-  lbm::CoupleArgs a{c->d_ccells, c->ncouple, c->d_cu, c->couple_rho ? c->d_crho : nullptr, c->couple_mode,
-                    c->couple_dt, c->cfg.tau, c->p64.omega};
+  const lbm::CoupleArgs a = lbm_couple_args(c);
   const lbm::BoundaryArgs bc{c->d_bct, c->d_bcu};
   const dim3 grid((unsigned)((c->ncouple + 255) / 256)), block(256);
   if (c->fp32) {
@@ -285,8 +207,7 @@ int lbm_enqueue_coupling_save(lbm_ctx* c) {
 // In-place layout: re-collide the coupled cells after the step of parity `parity` (0 even, 1 odd).
 int lbm_enqueue_coupling_aa(lbm_ctx* c, int parity) {
   if (!c->couple_on || c->ncouple == 0) return LBM_OK;
-  lbm::CoupleArgs a{c->d_ccells, c->ncouple, c->d_cu, c->couple_rho ? c->d_crho : nullptr, c->couple_mode,
-                    c->couple_dt, c->cfg.tau, c->p64.omega};
+  const lbm::CoupleArgs a = lbm_couple_args(c);
   const lbm::BoundaryArgs bc{c->d_bct, c->d_bcu};
   const dim3 grid((unsigned)((c->ncouple + 255) / 256)), block(256);
 #define LBM_COUPLE_AA(T, W, O)                                                                                   \
@@ -311,12 +232,15 @@ int lbm_enqueue_coupling_aa(lbm_ctx* c, int parity) {
 void lbm_coupling_release(lbm_ctx* c) {
   // captured steps hold the buffers' addresses: drop them before the buffers go
   if (c->d_ccells) lbm_graphs_release(c);
-  void* ptrs[] = {c->d_ccells, c->d_cu, c->d_crho, c->d_cout, c->d_csave};
+  void* ptrs[] = {c->d_ccells, c->d_cu, c->d_crho, c->d_cout, c->d_csave, c->d_cidx, c->d_cboxes};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   c->d_ccells = nullptr;
   c->d_cu = c->d_crho = c->d_cout = nullptr;
   c->d_csave = nullptr;
+  c->d_cidx = nullptr;
+  c->d_cboxes = nullptr;
+  c->ncboxes = 0;
   c->ncouple = 0;
   c->couple_on = false;
 }
@@ -335,11 +259,17 @@ int lbm_set_coupling_cells(lbm_ctx* c, const int64_t* cells, int64_t n) {
     if (cells[k] < 0 || cells[k] >= c->g.Nu) return cfail(c, LBM_ERR_ARG, "coupling cell out of range");
     if (seen[(size_t)cells[k]]++) return cfail(c, LBM_ERR_ARG, "coupling cells must be distinct");
   }
+  std::vector<int32_t> boxes;
+  if (!c->aa && n <= INT32_MAX) boxes = lbm::small_box_list(c->g, cells, n);
   if (lbm::device_alloc(&c->d_ccells, (size_t)n * sizeof(int64_t)) != hipSuccess ||
       lbm::device_alloc(&c->d_cu, (size_t)n * 3 * sizeof(double)) != hipSuccess ||
       lbm::device_alloc(&c->d_crho, (size_t)n * sizeof(double)) != hipSuccess ||
       lbm::device_alloc(&c->d_cout, (size_t)n * 4 * sizeof(double)) != hipSuccess ||
-      (c->aa && lbm::device_alloc(&c->d_csave, (size_t)n * Q * sizeof(double)) != hipSuccess)) {
+      (c->aa && lbm::device_alloc(&c->d_csave, (size_t)n * Q * sizeof(double)) != hipSuccess) ||
+      // sized for either cell order (lbm_set_flags may switch it)
+      (!boxes.empty() &&
+       (lbm::device_alloc(&c->d_cidx, (size_t)std::max(c->g_rows.N, c->g_bricks.N) * sizeof(int32_t)) != hipSuccess ||
+        lbm::device_alloc(&c->d_cboxes, boxes.size() * sizeof(int32_t)) != hipSuccess))) {
     lbm_coupling_release(c);
     return cfail(c, LBM_ERR_NOMEM, "coupling buffers allocation failed");
   }
@@ -356,6 +286,13 @@ int lbm_set_coupling_cells(lbm_ctx* c, const int64_t* cells, int64_t n) {
     return cfail(c, LBM_ERR_HIP, "coupling cell upload failed");
   }
   c->ncouple = n;
+  c->ncboxes = (int)boxes.size();
+  if ((!boxes.empty() &&
+       hipMemcpy(c->d_cboxes, boxes.data(), boxes.size() * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess) ||
+      lbm_couple_index(c) != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess) {
+    lbm_coupling_release(c);
+    return cfail(c, LBM_ERR_HIP, "coupling index failed");
+  }
   return LBM_OK;
 }
 
@@ -395,8 +332,7 @@ int lbm_get_coupling_data(lbm_ctx* c, double* u, double* rho) {
   if (!c->flags_set || !c->state_set) return cfail(c, LBM_ERR_STATE, "flags and state must be set first");
   if (hipSetDevice(c->cfg.device) != hipSuccess) return cfail(c, LBM_ERR_HIP, "hipSetDevice failed");
   const dim3 grid((unsigned)((c->ncouple + 255) / 256)), block(256);
-  const lbm::CoupleArgs a{c->d_ccells, c->ncouple, c->d_cu, c->couple_rho ? c->d_crho : nullptr, c->couple_mode,
-                          c->couple_dt, c->cfg.tau, c->p64.omega};
+  const lbm::CoupleArgs a = lbm_couple_args(c);
   const int on = c->couple_on ? 1 : 0;
   if (c->fp32)
     hipLaunchKernelGGL(lbm::k_couple_gather<float>, grid, block, 0, c->stream, lbm_state_geom(c), (const float*)c->buf[c->cur],

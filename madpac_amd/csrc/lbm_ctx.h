@@ -58,6 +58,9 @@ struct lbm_ctx {
   int64_t* d_ccells = nullptr;                  // coupled cells
   int64_t ncouple = 0;
   double *d_cu = nullptr, *d_crho = nullptr, *d_cout = nullptr;
+  int32_t* d_cidx = nullptr;                    // two-buffer layout: k of every coupled stored cell, else -1
+  int32_t* d_cboxes = nullptr;                  // ... and the boxes whose second step sees a coupled cell
+  int ncboxes = 0;
   double* d_csave = nullptr;                    // in-place layout: coupled cells' populations before a step
   bool couple_on = false, couple_rho = false;
   int couple_mode = 0;
@@ -95,6 +98,8 @@ int lbm_enqueue_coupling(lbm_ctx* c, const void* src, void* dst);
 // in-place layout: save the coupled cells' populations before a step, re-collide them after it
 int lbm_enqueue_coupling_save(lbm_ctx* c);
 int lbm_enqueue_coupling_aa(lbm_ctx* c, int parity);
+lbm::CoupleArgs lbm_couple_args(const lbm_ctx* c);
+hipError_t lbm_couple_index(lbm_ctx* c);  // d_cidx from d_ccells
 void lbm_coupling_release(lbm_ctx* c);
 void lbm_graphs_release(lbm_ctx* c);
 void lbm_adjoint_release(lbm_ctx* c);

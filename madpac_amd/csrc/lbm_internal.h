@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <string>
+#include <vector>
 
 #include "lbm_cell.h"
 
@@ -126,6 +127,17 @@ hipError_t launch_dense_step(const DenseGeom& g, bool fp32, bool f32math, const 
                              const uint32_t* words,
                              const void* alpha, bool force, bool walls, const CollideParams& p64,
                              const CollideParams32& p32, const BoundaryArgs& bc, bool spec, hipStream_t stream);
+// MD coupling of a context (lbm_couple.h)
+struct CoupleArgs {
+  const int64_t* cells;   // coupled cell indices
+  int64_t n;
+  const double* u;        // [3n] MD velocity (lattice units)
+  const double* rho;      // [n] MD density or null
+  int mode;               // LBM_COUPLE_*
+  double dt;              // LB time step of the Dirichlet forcing
+  double tau;             // configured tau (computeGi's _tau)
+  double omega;           // 1 / tau_eff (BlockBGK)
+};
 // Two steps src -> dst in one launch (lbm_pair.hip): the same state as two launch_dense_step.
 struct PairGeom {
   int tx, ty, tz;  // tiles of columns along x and y, chunks along z
@@ -134,8 +146,9 @@ struct PairGeom {
   int64_t passes;  // planes that one CU sweeps in sequence, pipeline fill included
 };
 // The split of this lattice, and whether launch_dense_pair takes it and is the faster way.
-// extra: force, porosity or boundary classes; open: classes other than moving walls.
-bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, PairGeom* plan);
+// extra: force, porosity or boundary classes; open: classes other than moving walls; coupled_boxes: boxes that
+// launch_coupled_boxes has to follow with (0: no coupling).
+bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, int coupled_boxes, PairGeom* plan);
 hipError_t launch_dense_pair(const DenseGeom& g, const PairGeom& plan, bool fp32, bool f32math, const void* src, void* dst,
                              const uint32_t* words, const void* alpha, bool force, bool walls, const CollideParams& p64,
                              const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t stream);
@@ -146,6 +159,14 @@ int small_steps(const DenseGeom& g);
 hipError_t launch_dense_small(const DenseGeom& g, int steps, bool fp32, bool f32math, const void* src, void* dst,
                               const uint32_t* words, const void* alpha, bool force, bool walls, const CollideParams& p64,
                               const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t stream);
+// Two steps src -> dst of the boxes listed (small_box_list) with the MD coupling, idx = the coupling's index of
+// every stored cell (-1: not coupled); no force and no porosity.
+hipError_t launch_coupled_boxes(const DenseGeom& g, bool fp32, bool f32math, const void* src, void* dst,
+                                const uint32_t* words, bool walls, const CollideParams& p64, const CollideParams32& p32,
+                                const BoundaryArgs& bc, const CoupleArgs& cpl, const int32_t* idx, const int32_t* boxes,
+                                int nboxes, hipStream_t stream);
+// The boxes of two steps that hold a listed cell (row-major) or a neighbour of one.
+std::vector<int32_t> small_box_list(const DenseGeom& g, const int64_t* cells, int64_t n);
 // reference state f (FP64) from the stored state
 // one in-place AA step on a single buffer: parity 0 reads the NATURAL layout and leaves SWAPPED,
 // parity 1 the reverse

@@ -355,8 +355,12 @@ hipError_t pair_type(const DenseGeom& g, const PairGeom& pg, bool fp32, bool f32
 // channel 189 / 240; 256^3 458 / 355, channel 502 / 530.  FP64 64^3 16.8 / 12.8, force and porosity 17.0 / 15.3,
 // lid 17.2 / 15.0, channel 16.2 / 19.3; 80^3 36.3 / 26.1, channel 38.1 / 39.1; 131 x 70 x 53 40.2 / 27.0,
 // channel 41.4 / 36.4; 256^3 932 / 527).  The microseconds of a plane are this table's.
+//  * With the MD coupling this kernel is followed by the boxes around the coupled cells (lbm_small.hip): 16 us
+//    and 45 ns a box (96^3 FP64: 14 us for 8 boxes, 23 for 216, 35 for 512, 173 for 3294), where a single step
+//    is followed by its re-collision, 7.5 us.  Per step, single / this way: 96^3 FP64 24^3 coupled cells 66.5 /
+//    52.3, 3000 scattered ones 74 / 127; 128^3 FP32 24^3 coupled cells 66.8 / 62.5.
 // A plane of populations has to fit the 32-bit offsets.
-bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, PairGeom* plan) {
+bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, int coupled_boxes, PairGeom* plan) {
   const int64_t plane = g.bricked ? (int64_t)64 * g.bnx * g.bny : (int64_t)g.nx * g.ny;
   if (plane * (g.aos ? Q : 1) * (int64_t)esize > (int64_t)UINT32_MAX) return false;
   const bool f64 = esize == 8;
@@ -368,7 +372,8 @@ bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, PairGeom
   }
   const double step = 3.0 + cells * 2 * Q * (double)esize / 5.3e6;
   const double pass = open ? 8.5 : f64 ? (extra ? 7.0 : 6.0) : (extra ? 5.7 : 5.1);
-  return (double)plan->passes * pass < 2.0 * step;
+  const double two = (double)plan->passes * pass;
+  return coupled_boxes ? two + 16.0 + 0.045 * coupled_boxes < 2.0 * (step + 7.5) : two < 2.0 * step;
 }
 
 hipError_t launch_dense_pair(const DenseGeom& g, const PairGeom& pg, bool fp32, bool f32math, const void* src, void* dst,

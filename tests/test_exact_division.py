@@ -40,3 +40,8 @@ def test_division_by_constants_is_correctly_rounded(divisor, z, zl):
     for x in xs:
         for v in (Fraction(x), -Fraction(x)):
             assert rounded(z * v + rounded(zl * v)) == rounded(v / c)
+
+
+def test_division_of_the_coupling_force_is_correctly_rounded():
+    # over_cs4: (c.u)^2 / ((1.0/3.0)*(1.0/3.0))
+    test_division_by_constants_is_correctly_rounded((1.0 / 3.0) * (1.0 / 3.0), 9.0, float.fromhex("0x1.2p-51"))
