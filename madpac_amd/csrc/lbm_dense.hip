@@ -15,6 +15,8 @@
 // BLB/nonlocaltreatment/AABlockStreaming.cpp:19-92); storing the post-collision state and
 // pulling gives the same numbers, because a moving-wall correction is applied to the outgoing
 // population of a wall link, which only that cell's own bounce-back ever reads.
+#include <type_traits>
+
 #include "lbm_collide.h"
 #include "lbm_geom.h"
 
@@ -41,6 +43,9 @@ DenseGeom make_geom(int nx, int ny, int nz, const int periodic[3], bool bricked,
   g.layout = LAYOUT_PULL;
   // interleaving needs whole 64-cell groups per brick or per row segment (addresses separable per axis)
   g.aos = (aos && (bricked || nx % BX == 0)) ? 1 : 0;
+  const double bytes = (double)Q * (double)g.N * (double)esize;
+  g.cached = state_cached(bytes) ? 1 : 0;
+  g.cached_pair = state_cached_pair(bytes) ? 1 : 0;
   return g;
 }
 
@@ -140,8 +145,15 @@ __global__ __launch_bounds__(BX * BY_MAX) void k_dense_step(DenseGeom g, const T
       for (int q = 0; q < Q; q++) f[q] = T(0);
     }
   }
+  if (g.cached) {
+    asm volatile("");
 #pragma unroll
-  for (int q = 0; q < Q; q++) __builtin_nontemporal_store(f[q], &dst[A.own(q)]);
+    for (int q = 0; q < Q; q++) dst[A.own(q)] = f[q];
+    asm volatile("");
+  } else {
+#pragma unroll
+    for (int q = 0; q < Q; q++) __builtin_nontemporal_store(f[q], &dst[A.own(q)]);
+  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -182,18 +194,25 @@ __global__ __launch_bounds__(BX * BY_MAX) void k_aa_step(DenseGeom g, T* __restr
   // addresses live through the collision (38 more VGPRs, one wave less per SIMD); an opaque copy
   // of the cell's base address makes it recompute them here instead.
   asm volatile("" : "+v"(A.base));
+  auto store = [&](auto cached) {
 #pragma unroll
-  for (int q = 0; q < Q; q++) {
-    // x + c_q is not fluid (a solid lane stores its zeros to its own slots)
-    const bool bounce = ((fl ? w : 0x7FFFFu) >> q) & 1u;
-    const int64_t di = (!ODD || bounce) ? A.own(Q - 1 - q) : A.push(q);
-    // An even step writes whole lines of its own slots.  An odd step's pushes fill each line from
-    // up to four wavefronts: ordinary stores let L2 merge the parts before write-back (measured
-    // 5-13 % faster on a porous 256^3 channel than streaming stores, which write each part out).
-    if (ODD)
-      a[di] = f[q];
-    else
-      __builtin_nontemporal_store(f[q], &a[di]);
+    for (int q = 0; q < Q; q++) {
+      // x + c_q is not fluid (a solid lane stores its zeros to its own slots)
+      const bool bounce = ((fl ? w : 0x7FFFFu) >> q) & 1u;
+      const int64_t di = (!ODD || bounce) ? A.own(Q - 1 - q) : A.push(q);
+      if constexpr (decltype(cached)::value) a[di] = f[q];
+      else __builtin_nontemporal_store(f[q], &a[di]);
+    }
+  };
+  // An even step writes whole lines of its own slots.  An odd step's pushes fill each line from
+  // up to four wavefronts: ordinary stores let L2 merge the parts before write-back (measured
+  // 5-13 % faster on a porous 256^3 channel than streaming stores, which write each part out).
+  if (ODD || g.cached) {
+    asm volatile("");
+    store(std::true_type{});
+    asm volatile("");
+  } else {
+    store(std::false_type{});
   }
 }
 
@@ -248,8 +267,15 @@ __global__ __launch_bounds__(BX * BY_MAX) void k_dense_copy(DenseGeom g, const T
   T f[Q];
 #pragma unroll
   for (int q = 0; q < Q; q++) f[q] = src[PULL ? A.pull(q) : A.own(q)];
+  if (g.cached) {
+    asm volatile("");
 #pragma unroll
-  for (int q = 0; q < Q; q++) __builtin_nontemporal_store(f[q], &dst[A.own(q)]);
+    for (int q = 0; q < Q; q++) dst[A.own(q)] = f[q];
+    asm volatile("");
+  } else {
+#pragma unroll
+    for (int q = 0; q < Q; q++) __builtin_nontemporal_store(f[q], &dst[A.own(q)]);
+  }
 }
 
 // The same state in another layout of the same cell order (e.g. pull form <-> AA NATURAL): each

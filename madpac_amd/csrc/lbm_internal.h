@@ -47,7 +47,20 @@ struct DenseGeom {
   int64_t nblocks_padded;    // rounded up to a multiple of NXCD
   int layout;                // how the stored state maps to the reference state (LAYOUT_*)
   int aos;                   // populations interleaved per group of 64 stored cells (pop_at)
+  int cached, cached_pair;   // 1: the steps (two-step kernel) store with ordinary stores, 0: past the caches
 };
+
+// Whether the steps' stores should go through the caches, by the bytes of the state: where it and its successor
+// stay in the 256 MB Infinity Cache from one step to the next.  Larger states only pass through it, and smaller
+// ones wait longer for the L2s' write-back between two launches than they gain.  One-step kernel, streaming /
+// ordinary stores, us: FP32 64 x 48 x 48 (11 MB) 8.1 / 9.1, 80^3 (39) 22.1 / 19.8, 96^3 (67) 30.9 / 25.7, 112^3 (107)
+// 52.9 / 35.6, 128^3 (159) 56.3 / 56.2, 160^3 (311) 119 / 125; FP64 48^3 (17) 10.2 / 10.5, 64^3 (40) 16.7 / 14.0,
+// 131 x 70 x 53 (74) 40.0 / 31.8, 96^3 (134) 58.9 / 56.8, 128 x 96 x 96 (179) 64.5 / 68.2.  In place, FP64 80^3
+// 34.1 / 30.9, 96^3 52.6 / 48.7.  Two-step kernel, a step: FP64 64^3 12.5 / 12.7, 131 x 70 x 53 26.8 / 21.8, 96^3
+// 38.0 / 35.2, 128 x 96 x 96 44.9 / 46.5; FP32 128^3 47.3 / 49.8.  (A branch with both kinds of store needs
+// something between them: the compiler merges them into ordinary ones.)
+inline bool state_cached(double bytes) { return bytes >= 20e6 && bytes <= 140e6; }
+inline bool state_cached_pair(double bytes) { return bytes >= 60e6 && bytes <= 140e6; }
 
 // Address of population q of stored cell i in a state buffer.  Planes (aos = 0): plane q holds
 // population q of every cell, q * N + i.  Interleaved (aos = 1): the 19 populations of each group
@@ -146,9 +159,11 @@ struct PairGeom {
   int64_t passes;  // planes that one CU sweeps in sequence, pipeline fill included
 };
 // The split of this lattice, and whether launch_dense_pair takes it and is the faster way.
-// extra: force, porosity or boundary classes; open: classes other than moving walls; coupled_boxes: boxes that
+// extra: force or porosity; walls: boundary classes; open: classes other than moving walls; coupled_boxes: boxes that
 // launch_coupled_boxes has to follow with (0: no coupling).
-bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, int coupled_boxes, PairGeom* plan);
+// nfluid: fluid cells.
+bool pair_plan(const DenseGeom& g, size_t esize, int64_t nfluid, bool extra, bool walls, bool open, int coupled_boxes,
+               PairGeom* plan);
 hipError_t launch_dense_pair(const DenseGeom& g, const PairGeom& plan, bool fp32, bool f32math, const void* src, void* dst,
                              const uint32_t* words, const void* alpha, bool force, bool walls, const CollideParams& p64,
                              const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t stream);

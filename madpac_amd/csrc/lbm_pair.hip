@@ -254,8 +254,15 @@ __global__ __launch_bounds__((Tile<TX, TY>::THREADS), 3) void k_dense_pair(
     if (out && act && (fl || line_has_fluid<T>(fluid))) {
       if (fl) collide_cell_bc<T, FORCE, ALPHA, WALLS, M32>(h, wp, cell_z(p) + cell_xy, alpha, p64, p32, bc);
       T* dz = dst + term_z(p);
+      if (g.cached_pair) {
+        asm volatile("");
 #pragma unroll
-      for (int q = 0; q < Q; q++) __builtin_nontemporal_store(fl ? h[q] : T(0), (T*)((char*)(dz + pop(q)) + col[1][1]));
+        for (int q = 0; q < Q; q++) *(T*)((char*)(dz + pop(q)) + col[1][1]) = fl ? h[q] : T(0);
+        asm volatile("");
+      } else {
+#pragma unroll
+        for (int q = 0; q < Q; q++) __builtin_nontemporal_store(fl ? h[q] : T(0), (T*)((char*)(dz + pop(q)) + col[1][1]));
+      }
     }
     r16 = ((wc >> 2) & 1u) ? c2 : s16;
     r9 = c9;
@@ -345,33 +352,36 @@ hipError_t pair_type(const DenseGeom& g, const PairGeom& pg, bool fp32, bool f32
 }  // namespace
 
 // The rule weighs two launches of the one-step kernel against one of this kernel, in microseconds.
-//  * One step: 3 and its bytes at 5.3 TB/s, with half of the lanes that rows leave idle, and a fifth more
-//    where rows do not start on 128-byte lines.
+//  * One step: 3, a boundary's 1, and its bytes at 5.3 TB/s (7 where the caches hold them, state_cached), with half
+//    of the lanes that rows leave idle, and a fifth more where rows do not start on 128-byte lines; of the
+//    solid cells' bytes a half (where the caches hold them, none).
 //  * This kernel: its planes in sequence (PairGeom::passes), each a latency: loads, two collisions, two
 //    barriers.  Force, porosity and boundary classes lengthen the collisions, open boundaries most: their
 //    cells' two equilibria per link hold up the whole workgroup.
-// Measured per step, one-step / this kernel (FP32 96^3 periodic 30.9 / 31.4, force and porosity 30.7 / 37.8, lid
-// 31.8 / 36.8, channel 35.2 / 48.4; 128^3 55.3 / 46.7, force and porosity 56.6 / 54.2; 192^3 187 / 167,
-// channel 189 / 240; 256^3 458 / 355, channel 502 / 530.  FP64 64^3 16.8 / 12.8, force and porosity 17.0 / 15.3,
-// lid 17.2 / 15.0, channel 16.2 / 19.3; 80^3 36.3 / 26.1, channel 38.1 / 39.1; 131 x 70 x 53 40.2 / 27.0,
-// channel 41.4 / 36.4; 256^3 932 / 527).  The microseconds of a plane are this table's.
+// Measured per step, one-step / this kernel: FP32 96^3 periodic 25.9 / 29, lid 27.8 / 35, channel 30.5 / 47;
+// 112^3 35.6 / 37.5; 128^3 55.3 / 46.7, force and porosity 56.6 / 54.2; 192^3 187 / 167, channel 189 / 240; 256^3 458 /
+// 355, channel 502 / 530.  FP64 64^3 14.2 / 12.7, force and porosity 14.0 / 14.8, lid 15.3 / 14.7; 80^3 30.9 / 23.5,
+// channel 30.7 / 38; 131 x 70 x 53 31.8 / 21.8, channel 31.6 / 32.0; 256^3 932 / 527.  The microseconds of a plane
+// are this table's.
 //  * With the MD coupling this kernel is followed by the boxes around the coupled cells (lbm_small.hip): 16 us
 //    and 45 ns a box (96^3 FP64: 14 us for 8 boxes, 23 for 216, 35 for 512, 173 for 3294), where a single step
 //    is followed by its re-collision, 7.5 us.  Per step, single / this way: 96^3 FP64 24^3 coupled cells 66.5 /
 //    52.3, 3000 scattered ones 74 / 127; 128^3 FP32 24^3 coupled cells 66.8 / 62.5.
 // A plane of populations has to fit the 32-bit offsets.
-bool pair_plan(const DenseGeom& g, size_t esize, bool extra, bool open, int coupled_boxes, PairGeom* plan) {
+bool pair_plan(const DenseGeom& g, size_t esize, int64_t nfluid, bool extra, bool walls, bool open, int coupled_boxes,
+               PairGeom* plan) {
   const int64_t plane = g.bricked ? (int64_t)64 * g.bnx * g.bny : (int64_t)g.nx * g.ny;
   if (plane * (g.aos ? Q : 1) * (int64_t)esize > (int64_t)UINT32_MAX) return false;
   const bool f64 = esize == 8;
   *plan = f64 && g.bricked ? pair_geom(g, 32, 16) : pair_geom(g, 64, 8);
-  double cells = (double)g.Nu;
+  const bool held = g.cached && (double)Q * (double)g.N * (double)esize <= 125e6;
+  double cells = held ? (double)nfluid : 0.5 * ((double)nfluid + (double)g.Nu);
   if (!g.bricked) {
     cells *= 0.5 + 0.5 * ((g.nx + 63) / 64 * 64) / g.nx;
     if ((g.nx * esize) % 128) cells *= 1.2;
   }
-  const double step = 3.0 + cells * 2 * Q * (double)esize / 5.3e6;
-  const double pass = open ? 8.5 : f64 ? (extra ? 7.0 : 6.0) : (extra ? 5.7 : 5.1);
+  const double step = 3.0 + (walls ? 1.0 : 0.0) + cells * 2 * Q * (double)esize / (held ? 7.0e6 : 5.3e6);
+  const double pass = open ? (f64 ? 8.0 : 8.5) : extra ? (f64 ? 6.2 : 5.7) : walls ? (f64 ? 5.9 : 5.7) : (f64 ? 5.2 : 5.1);
   const double two = (double)plan->passes * pass;
   return coupled_boxes ? two + 16.0 + 0.045 * coupled_boxes < 2.0 * (step + 7.5) : two < 2.0 * step;
 }

@@ -178,7 +178,7 @@ __device__ __forceinline__ int pull_slot(int q, const PatchLane& L) {
 template <typename T, bool M32, bool FL>
 __device__ __forceinline__ void patch_cell(const PatchDev* __restrict__ pp, const uint32_t* __restrict__ words,
                                            const T* __restrict__ s, T* __restrict__ d, T* __restrict__ dst, int n,
-                                           double omega, int x, int y, int z) {
+                                           double omega, int x, int y, int z, bool cached) {
   T f[Q];
   uint32_t w = 0u;
   {
@@ -198,8 +198,15 @@ __device__ __forceinline__ void patch_cell(const PatchDev* __restrict__ pp, cons
   // they cost more registers than the collision leaves (spills).
   asm volatile("" : "+v"(x), "+v"(y), "+v"(z));
   const PatchLane L = patch_lane(n, x, y, z);
+  if (cached) {
+    asm volatile("");
 #pragma unroll
-  for (int q = 0; q < Q; q++) __builtin_nontemporal_store(f[q], &d[q * L.n3 + L.i]);
+    for (int q = 0; q < Q; q++) d[q * L.n3 + L.i] = f[q];
+    asm volatile("");
+  } else {
+#pragma unroll
+    for (int q = 0; q < Q; q++) __builtin_nontemporal_store(f[q], &d[q * L.n3 + L.i]);
+  }
   if (L.lx | L.hx | L.ly | L.hy | L.lz | L.hz) {
     const int n2 = L.n2, G0 = Q * L.n3, E0 = G0 + 30 * n2;
 #pragma unroll
@@ -242,7 +249,7 @@ template <typename T, int TX, int TY, int TZ, bool M32, bool FL, bool CHUNK>
 __global__ __launch_bounds__(256) void k_patch_step(const PatchDev* __restrict__ patches,
                                                     const TileDev* __restrict__ tiles, int ntiles,
                                                     const uint32_t* __restrict__ words,
-                                                    const T* __restrict__ src, T* __restrict__ dst) {
+                                                    const T* __restrict__ src, T* __restrict__ dst, bool cached) {
   constexpr int TC = TX * TY * TZ;
   int t, end, stride;
   tile_range<CHUNK>(ntiles, t, end, stride);
@@ -259,7 +266,7 @@ __global__ __launch_bounds__(256) void k_patch_step(const PatchDev* __restrict__
     for (int c = threadIdx.x; c < TC; c += 256) {
       const int x = tl.x0 + c % TX, y = tl.y0 + (c / TX) % TY, z = tl.z0 + c / (TX * TY);
       if (x >= n || y >= n || z >= n) continue;
-      patch_cell<T, M32, FL>(pp, words, src + tl.base, dst + tl.base, dst, n, tl.omega, x, y, z);
+      patch_cell<T, M32, FL>(pp, words, src + tl.base, dst + tl.base, dst, n, tl.omega, x, y, z, cached);
     }
     if (tn >= end) break;
     t = tn;
@@ -288,7 +295,7 @@ template <typename T, bool M32, bool FL, bool CHUNK>
 __global__ __launch_bounds__(256, patch_waves_per_simd<T>()) void k_patch_step_lin(const PatchDev* __restrict__ patches,
                                                         const TileDev* __restrict__ tiles, int ntiles,
                                                         const uint32_t* __restrict__ words,
-                                                        const T* __restrict__ src, T* __restrict__ dst) {
+                                                        const T* __restrict__ src, T* __restrict__ dst, bool cached) {
   int t, end, stride;
   tile_range<CHUNK>(ntiles, t, end, stride);
   if (t >= end) return;
@@ -310,7 +317,7 @@ __global__ __launch_bounds__(256, patch_waves_per_simd<T>()) void k_patch_step_l
         case 32: split_cell<32>(c, n, x, y, z); break;
         default: split_cell<0>(c, n, x, y, z); break;
       }
-      patch_cell<T, M32, FL>(pp, words, src + tl.base, dst + tl.base, dst, n, tl.omega, x, y, z);
+      patch_cell<T, M32, FL>(pp, words, src + tl.base, dst + tl.base, dst, n, tl.omega, x, y, z, cached);
     }
     if (tn >= end) break;
     t = tn;
@@ -627,10 +634,11 @@ hipError_t launch_step_c(lbm_patchset* ps, const void* src, void* dst) {
   const dim3 grid((unsigned)std::max(1, wgs)), block(256);
   const T* s = (const T*)src;
   T* d = (T*)dst;
+  const bool cached = state_cached((double)ps->elems * (double)ps->esize);
 #define LBM_PATCH(X, Y, Z)                                                                                     \
   if (t.tile_x == X && t.tile_y == Y && t.tile_z == Z) {                                                       \
     hipLaunchKernelGGL((k_patch_step<T, X, Y, Z, M32, FL, CHUNK>), grid, block, 0, ps->stream, ps->d_patches,   \
-                       ps->d_tiles, ps->ntiles, ps->d_words, s, d);                                            \
+                       ps->d_tiles, ps->ntiles, ps->d_words, s, d, cached);                                            \
     return hipGetLastError();                                                                                  \
   }
   LBM_PATCH(8, 8, 4)
@@ -641,7 +649,7 @@ hipError_t launch_step_c(lbm_patchset* ps, const void* src, void* dst) {
 #undef LBM_PATCH
   if (linear_tiles(t)) {
     hipLaunchKernelGGL((k_patch_step_lin<T, M32, FL, CHUNK>), grid, block, 0, ps->stream, ps->d_patches,
-                       ps->d_tiles, ps->ntiles, ps->d_words, s, d);
+                       ps->d_tiles, ps->ntiles, ps->d_words, s, d, cached);
     return hipGetLastError();
   }
   return hipErrorInvalidValue;
