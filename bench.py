@@ -45,6 +45,11 @@ def read_traffic(key):
     return None
 
 
+def steps_per_launch(lbm, n, layout, steps):
+    """Two-buffer lattices of 128^3 cells and more without open boundaries advance two steps per launch."""
+    return 2 if layout == lbm.LAYOUT_TWO_BUFFER and steps >= 2 and n >= 128 else 1
+
+
 def run_dense(lbm, solid, n, tau, prec, steps, warmup, g, layout=0, readout=False):
     lat = lbm.Lattice(n, n, n, tau, precision=prec, periodic=(True, True, True), force=(g, 0.0, 0.0), layout=layout)
     lat.set_flags(~solid)
@@ -55,7 +60,7 @@ def run_dense(lbm, solid, n, tau, prec, steps, warmup, g, layout=0, readout=Fals
     lat.step(warmup)
     lat.synchronize()
     t0 = time.perf_counter()
-    ms = lat.step_timed(steps)  # HIP events on the context stream around exactly `steps` launches
+    ms = lat.step_timed(steps)  # HIP events on the context stream around exactly `steps` steps
     lat.synchronize()
     wall = time.perf_counter() - t0
     ceil = None
@@ -81,15 +86,20 @@ def run_dense(lbm, solid, n, tau, prec, steps, warmup, g, layout=0, readout=Fals
                 "populations_s": round(t2 - t1, 4), "populations_bytes": n ** 3 * 19 * 8}
     lat.close()
     esize = 8 if prec == lbm.FP64 else 4
-    per_launch_s = ms * 1e-3 / steps
+    # The two-buffer lattice of this size runs two steps per launch: one read and one write of the state for both.
+    # `achieved` counts the bytes that a launch has to move; `one_step` the 38 values of every update, which a
+    # one-step kernel would have to move (it can exceed what HBM carries).
+    per_launch = steps_per_launch(lbm, n, layout, steps)
     bytes_per_launch = nfluid * 2 * 19 * esize
-    achieved = bytes_per_launch / per_launch_s / 1e9
+    achieved = bytes_per_launch / (ms * 1e-3 / steps * per_launch) / 1e9
     schedule = "aa-in-place" if layout == lbm.LAYOUT_AA else ("loads-with-flag-word" if variant & 1 else "flag-word-first")
     dispatch = "xcd-contiguous" if variant & 2 else "dispatch-order"
     shape = (variant >> 2) & 3
     # the shape bits are 0 only when the tuner could not copy the state: then the default holds
     wg_rows = (2, 4, 8)[shape - 1] if shape else 4
     key = f"{'fp64' if prec == lbm.FP64 else 'fp32s'} {n}^3 {schedule} ({wg_rows} {order}/workgroup)"
+    if per_launch == 2:
+        key = f"{'fp64' if prec == lbm.FP64 else 'fp32s'} {n}^3 two steps per launch ({order})"
     traffic = read_traffic(key)
     return {
         "mlups": nfluid * steps / (ms * 1e-3) / 1e6,
@@ -106,15 +116,17 @@ def run_dense(lbm, solid, n, tau, prec, steps, warmup, g, layout=0, readout=Fals
         "copy_reference": ceil,
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "algorithmic_bytes_per_launch": bytes_per_launch},
+                     "algorithmic_bytes_per_launch": bytes_per_launch, "steps_per_launch": per_launch,
+                     "one_step": {"GBs": round(achieved * per_launch, 1),
+                                  "frac": round(achieved * per_launch / HBM_PEAK_GBS, 4)}},
     }
 
 
 def run_md_coupling(lbm, solid, n, tau, steps=100, box=40):
     """The MD coupling hooks (PeanoDataExchangeService.cpp:69-218) on the porous channel's geometry
     without its body force (coupled cells take the plain BGK collision, which the library enforces),
-    FP64: the fluid cells of a box^3 MD region in the middle of the lattice are coupled in Dirichlet mode (after
-    the step kernel, k_couple re-collides them with the MD velocity); the step with coupling against
+    FP64: the fluid cells of a box^3 MD region in the middle of the lattice are coupled in Dirichlet mode (two
+    steps per launch, then the boxes around the coupled cells once more with the MD velocity); the step with coupling against
     the same step without it, both timed with HIP events on the context stream, and the export of the
     region's density and velocity (k_couple_gather plus the copy to host memory, wall clock)."""
     lo = (n - box) // 2
@@ -160,9 +172,10 @@ def run_taylor_green(lbm, wl, n=512, steps=200, tau=0.52, u0=0.04):
             lat.step(10)
             ms = lat.step_timed(steps) / steps
         esize = 8 if prec == lbm.FP64 else 4
-        gbs = n ** 3 * 38 * esize / (ms * 1e-3) / 1e9
+        k = steps_per_launch(lbm, n, lbm.LAYOUT_TWO_BUFFER, steps)
+        gbs = n ** 3 * 38 * esize / (k * ms * 1e-3) / 1e9  # the state read and written once per launch
         out[name] = {"value": round(n ** 3 / (ms * 1e3), 1), "unit": "MLUPS", "ms_per_step": round(ms, 4),
-                     "roofline_frac": round(gbs / HBM_PEAK_GBS, 4)}
+                     "steps_per_launch": k, "roofline_frac": round(gbs / HBM_PEAK_GBS, 4)}
     return out
 
 
@@ -185,7 +198,8 @@ def run_shard_share(lbm, solid, tau, g, planes=32, steps=300):
             order = "bricks" if lat.cell_order == lbm.CELL_ORDER_BRICKS else "rows"
         esize = 8 if prec == lbm.FP64 else 4
         out[name] = {"value": round(nfl / (ms * 1e3), 1), "unit": "MLUPS", "ms_per_step": round(ms, 4),
-                     "roofline_frac": round(nfl * 38 * esize / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+                     "steps_per_launch": 2,  # 2.2 M cells: two steps per launch in both precisions
+                     "roofline_frac": round(nfl * 38 * esize / (2 * ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                      "cell_order": order}
     return out
 
