@@ -153,6 +153,7 @@ struct CoupleArgs {
 };
 // Two steps src -> dst in one launch (lbm_pair.hip): the same state as two launch_dense_step.
 struct PairGeom {
+  int tile_x;      // 64 (tiles of 64 x 8 columns) or 32 (32 x 16)
   int tx, ty, tz;  // tiles of columns along x and y, chunks along z
   int cz;          // planes per chunk
   int64_t nblocks, nblocks_padded;

@@ -286,6 +286,7 @@ constexpr int NCU = 256;
 
 PairGeom pair_geom(const DenseGeom& g, int tile_x, int tile_y) {
   PairGeom p;
+  p.tile_x = tile_x;
   p.tx = (g.nx + tile_x - 1) / tile_x;
   p.ty = (g.ny + tile_y - 1) / tile_y;
   const int64_t tiles = (int64_t)p.tx * p.ty;
@@ -332,10 +333,8 @@ template <typename T, bool M32, bool AOS>
 hipError_t pair_tile(const DenseGeom& g, const PairGeom& pg, const void* src, void* dst, const uint32_t* words, const void* alpha, bool force,
                      bool walls, const CollideParams& p64, const CollideParams32& p32, const BoundaryArgs& bc,
                      hipStream_t s) {
-  if constexpr (sizeof(T) == 8) {
-    if (g.bricked)
-      return pair_t<T, M32, AOS, 32, 16>(g, pg, src, dst, words, alpha, force, walls, p64, p32, bc, s);
-  }
+  if (pg.tile_x == 32)
+    return pair_t<T, M32, AOS, 32, 16>(g, pg, src, dst, words, alpha, force, walls, p64, p32, bc, s);
   return pair_t<T, M32, AOS, 64, 8>(g, pg, src, dst, words, alpha, force, walls, p64, p32, bc, s);
 }
 
@@ -367,13 +366,20 @@ hipError_t pair_type(const DenseGeom& g, const PairGeom& pg, bool fp32, bool f32
 //    and 45 ns a box (96^3 FP64: 14 us for 8 boxes, 23 for 216, 35 for 512, 173 for 3294), where a single step
 //    is followed by its re-collision, 7.5 us.  Per step, single / this way: 96^3 FP64 24^3 coupled cells 66.5 /
 //    52.3, 3000 scattered ones 74 / 127; 128^3 FP32 24^3 coupled cells 66.8 / 62.5.
+//  * Two tiles of 512 columns, 64 x 8 and 32 x 16; where both need as many planes 64 x 8 is the faster one
+//    by 5 % (32 x 16 in FP64 bricks, by 4 %: head of this file), but rows of 80, 96 or 160 cells leave it half
+//    empty at their end.  A step in 64 x 8 / 32 x 16: FP64 80^3 force and porosity 30.8 / 24.4, 96^3 (13 and 10
+//    planes) lid 40.0 / 34.5, channel 50.9 / 42.3, 160^3 (43 and 35) 155 / 145; FP32 160^3 118 / 105.
 // A plane of populations has to fit the 32-bit offsets.
 bool pair_plan(const DenseGeom& g, size_t esize, int64_t nfluid, bool extra, bool walls, bool open, int coupled_boxes,
                PairGeom* plan) {
   const int64_t plane = g.bricked ? (int64_t)64 * g.bnx * g.bny : (int64_t)g.nx * g.ny;
   if (plane * (g.aos ? Q : 1) * (int64_t)esize > (int64_t)UINT32_MAX) return false;
   const bool f64 = esize == 8;
-  *plan = f64 && g.bricked ? pair_geom(g, 32, 16) : pair_geom(g, 64, 8);
+  const PairGeom wide = pair_geom(g, 64, 8), tall = pair_geom(g, 32, 16);
+  const bool bricks = f64 && g.bricked;
+  const double t_wide = (double)wide.passes * (bricks ? 1.04 : 1.0), t_tall = (double)tall.passes * (bricks ? 1.0 : 1.05);
+  *plan = t_tall < t_wide ? tall : wide;
   const bool held = g.cached && (double)Q * (double)g.N * (double)esize <= 125e6;
   double cells = held ? (double)nfluid : 0.5 * ((double)nfluid + (double)g.Nu);
   if (!g.bricked) {
@@ -382,7 +388,7 @@ bool pair_plan(const DenseGeom& g, size_t esize, int64_t nfluid, bool extra, boo
   }
   const double step = 3.0 + (walls ? 1.0 : 0.0) + cells * 2 * Q * (double)esize / (held ? 7.0e6 : 5.3e6);
   const double pass = open ? (f64 ? 8.0 : 8.5) : extra ? (f64 ? 6.2 : 5.7) : walls ? (f64 ? 5.9 : 5.7) : (f64 ? 5.2 : 5.1);
-  const double two = (double)plan->passes * pass;
+  const double two = std::min(t_wide, t_tall) * pass;
   return coupled_boxes ? two + 16.0 + 0.045 * coupled_boxes < 2.0 * (step + 7.5) : two < 2.0 * step;
 }
 

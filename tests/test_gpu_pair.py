@@ -83,3 +83,18 @@ def test_pairs_in_a_captured_graph():
 def test_pairs_equal_single_steps_where_they_pay(size, scene, prec, order):
     # sizes that the rule of pair_plan sends to the two-step kernel, with each kind of boundary it weighs
     test_pairs_equal_single_steps(size, scene, prec, order)
+
+
+@pytest.mark.parametrize("size, scene, prec, order", [
+    ((95, 97, 83), "porous", lbm.FP64, ROWS),                # one idle lane, last tile of one row
+    ((160, 81, 66), "channel", lbm.FP64, ROWS),              # whole tiles along x, inlet and outlet
+    ((96, 90, 88), "cavity", lbm.FP64, ROWS),
+    ((159, 147, 150), "brinkman", lbm.FP32_SHIFTED, ROWS),   # last tile of three rows
+    ((96, 161, 149), "open", lbm.FP32_SHIFTED, ROWS),        # last tile of one row, wrapping axes
+    ((160, 158, 150), "cavity", lbm.FP32_SHIFTED, ROWS),
+    ((93, 177, 180), "porous", lbm.FP32_SHIFTED, BRICKS),    # bricks cut by the box
+    ((130, 120, 118), "porous", lbm.FP32_SHIFTED_F32, ROWS),  # last tile of two columns
+])
+def test_pairs_in_tall_tiles_equal_single_steps(size, scene, prec, order):
+    # sizes that fill tiles of 32 x 16 columns better than those of 64 x 8
+    test_pairs_equal_single_steps(size, scene, prec, order)
