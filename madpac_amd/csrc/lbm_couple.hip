@@ -259,19 +259,24 @@ int lbm_set_coupling_cells(lbm_ctx* c, const int64_t* cells, int64_t n) {
     if (cells[k] < 0 || cells[k] >= c->g.Nu) return cfail(c, LBM_ERR_ARG, "coupling cell out of range");
     if (seen[(size_t)cells[k]]++) return cfail(c, LBM_ERR_ARG, "coupling cells must be distinct");
   }
-  std::vector<int32_t> boxes;
-  if (!c->aa && n <= INT32_MAX) boxes = lbm::small_box_list(c->g, cells, n);
   if (lbm::device_alloc(&c->d_ccells, (size_t)n * sizeof(int64_t)) != hipSuccess ||
       lbm::device_alloc(&c->d_cu, (size_t)n * 3 * sizeof(double)) != hipSuccess ||
       lbm::device_alloc(&c->d_crho, (size_t)n * sizeof(double)) != hipSuccess ||
       lbm::device_alloc(&c->d_cout, (size_t)n * 4 * sizeof(double)) != hipSuccess ||
-      (c->aa && lbm::device_alloc(&c->d_csave, (size_t)n * Q * sizeof(double)) != hipSuccess) ||
-      // sized for either cell order (lbm_set_flags may switch it)
-      (!boxes.empty() &&
-       (lbm::device_alloc(&c->d_cidx, (size_t)std::max(c->g_rows.N, c->g_bricks.N) * sizeof(int32_t)) != hipSuccess ||
-        lbm::device_alloc(&c->d_cboxes, boxes.size() * sizeof(int32_t)) != hipSuccess))) {
+      (c->aa && lbm::device_alloc(&c->d_csave, (size_t)n * Q * sizeof(double)) != hipSuccess)) {
     lbm_coupling_release(c);
     return cfail(c, LBM_ERR_NOMEM, "coupling buffers allocation failed");
+  }
+  // for pairs of steps; without room for the index (sized for either cell order, as lbm_set_flags may switch
+  // it) coupled runs take single steps
+  std::vector<int32_t> boxes;
+  if (!c->aa && n <= INT32_MAX) boxes = lbm::small_box_list(c->g, cells, n);
+  if (!boxes.empty() &&
+      (lbm::device_alloc(&c->d_cidx, (size_t)std::max(c->g_rows.N, c->g_bricks.N) * sizeof(int32_t)) != hipSuccess ||
+       lbm::device_alloc(&c->d_cboxes, boxes.size() * sizeof(int32_t)) != hipSuccess)) {
+    if (c->d_cidx) (void)hipFree(c->d_cidx);
+    c->d_cidx = nullptr;
+    boxes.clear();
   }
   // the kernels address the stored (bricked) cells
   const lbm::DenseGeom& g = c->g;
