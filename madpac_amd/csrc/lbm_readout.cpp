@@ -10,9 +10,9 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -122,7 +122,7 @@ hipError_t through_ring(Staging& r, const HostCopy* parts, int nparts, hipStream
   for (int t = 0; t < want; t++) {
     try {
       threads.emplace_back(worker);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {  // no thread or no memory for one: those that run move all pieces
       break;
     }
   }
@@ -160,7 +160,7 @@ hipError_t read_back(const HostCopy* parts, int n, hipStream_t stream) {
       hipError_t e;
       try {
         e = through_ring(*r, parts, n, stream);
-      } catch (const std::bad_alloc&) {  // before any thread is started
+      } catch (const std::bad_alloc&) {  // from the lists, before any thread is started
         e = hipErrorOutOfMemory;
       }
       (void)hipStreamSynchronize(stream);  // nothing is on its way into the ring when it is given back
