@@ -168,6 +168,7 @@ int lbm_create(lbm_ctx** out, const lbm_config* cfg) {
   c->g_rows = lbm::make_geom(cfg->nx, cfg->ny, cfg->nz, cfg->periodic, false, c->esize, aos);
   c->g_bricks = lbm::make_geom(cfg->nx, cfg->ny, cfg->nz, cfg->periodic, true, c->esize, aos);
   c->g = cfg->cell_order == LBM_CELL_ORDER_BRICKS ? c->g_bricks : c->g_rows;
+  c->splits = lbm::pair_splits(c->g);
   c->force = cfg->force[0] != 0.0 || cfg->force[1] != 0.0 || cfg->force[2] != 0.0;
   c->p64.tau_eff = lbm_tau_effective(cfg->tau);
   c->p64.omega = 1.0 / c->p64.tau_eff;
@@ -508,7 +509,9 @@ StepPlan plan_steps(const lbm_ctx* c) {
   if (p.small) return p;
   bool open = false;
   for (const lbm::BoundaryClass& b : c->bct) open = open || (b.mask && (b.type & lbm::BC_TYPE_MASK) != lbm::BC_MOVING_WALL);
-  if (lbm::pair_plan(c->g, c->esize, c->nfluid, c->force || c->alpha, c->walls, open, p.coupled ? c->ncboxes : 0, &p.pair)) p.most = 2;
+  if (lbm::pair_plan(c->g, c->splits, c->esize, c->nfluid, c->force || c->alpha, c->walls, open,
+                     p.coupled ? c->ncboxes : 0, &p.pair))
+    p.most = 2;
   return p;
 }
 

@@ -33,6 +33,7 @@ struct lbm_ctx {
   lbm_config cfg{};
   lbm::DenseGeom g{};                  // geometry of the cell order in use (one of the two below)
   lbm::DenseGeom g_rows{}, g_bricks{};
+  lbm::PairSplits splits{};            // tiles and chunks of the two-step kernel (the same for both orders)
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::string err;

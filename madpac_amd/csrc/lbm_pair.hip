@@ -350,6 +350,8 @@ hipError_t pair_type(const DenseGeom& g, const PairGeom& pg, bool fp32, bool f32
 
 }  // namespace
 
+PairSplits pair_splits(const DenseGeom& g) { return PairSplits{pair_geom(g, 64, 8), pair_geom(g, 32, 16)}; }
+
 // The rule weighs two launches of the one-step kernel against one of this kernel, in microseconds.
 //  * One step: 3, a boundary's 1, and its bytes at 5.3 TB/s (7 where the caches hold them, state_cached), with half
 //    of the lanes that rows leave idle, and a fifth more where rows do not start on 128-byte lines; of the
@@ -371,12 +373,12 @@ hipError_t pair_type(const DenseGeom& g, const PairGeom& pg, bool fp32, bool f32
 //    empty at their end.  A step in 64 x 8 / 32 x 16: FP64 80^3 force and porosity 30.8 / 24.4, 96^3 (13 and 10
 //    planes) lid 40.0 / 34.5, channel 50.9 / 42.3, 160^3 (43 and 35) 155 / 145; FP32 160^3 118 / 105.
 // A plane of populations has to fit the 32-bit offsets.
-bool pair_plan(const DenseGeom& g, size_t esize, int64_t nfluid, bool extra, bool walls, bool open, int coupled_boxes,
-               PairGeom* plan) {
+bool pair_plan(const DenseGeom& g, const PairSplits& splits, size_t esize, int64_t nfluid, bool extra, bool walls,
+               bool open, int coupled_boxes, PairGeom* plan) {
   const int64_t plane = g.bricked ? (int64_t)64 * g.bnx * g.bny : (int64_t)g.nx * g.ny;
   if (plane * (g.aos ? Q : 1) * (int64_t)esize > (int64_t)UINT32_MAX) return false;
   const bool f64 = esize == 8;
-  const PairGeom wide = pair_geom(g, 64, 8), tall = pair_geom(g, 32, 16);
+  const PairGeom &wide = splits.wide, &tall = splits.tall;
   const bool bricks = f64 && g.bricked;
   const double t_wide = (double)wide.passes * (bricks ? 1.04 : 1.0), t_tall = (double)tall.passes * (bricks ? 1.0 : 1.05);
   *plan = t_tall < t_wide ? tall : wide;
