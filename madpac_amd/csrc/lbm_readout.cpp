@@ -82,6 +82,15 @@ void give_ring(Staging* r) {
   if (g_holders == 0) free_ring(*r);
 }
 
+// Memory that the runtime knows (pinned above all) takes the transfer itself: rho and u of 256^3 cells into
+// pinned memory 10.0 ms, through the ring 14.0; 96^3 0.56 and 0.97.
+bool known(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return false;
+}
+
 struct Piece {
   char* dst;
   const char* src;
@@ -153,22 +162,32 @@ hipError_t through_ring(Staging& r, const HostCopy* parts, int nparts, hipStream
 }  // namespace
 
 hipError_t read_back(const HostCopy* parts, int n, hipStream_t stream) {
-  size_t total = 0;
+  constexpr int MOST = 4;
+  HostCopy staged[MOST];
+  int nstaged = 0;
+  size_t total = 0, large = 0;
   for (int p = 0; p < n; p++) total += parts[p].bytes;
-  if (total >= DIRECT) {
+  for (int p = 0; p < n && n <= MOST && total >= DIRECT; p++)
+    if (!known(parts[p].dst)) {
+      staged[nstaged++] = parts[p];
+      large += parts[p].bytes;
+    }
+  bool arrived = false;  // the staged parts
+  if (large >= DIRECT) {
     if (Staging* r = take_ring()) {
       hipError_t e;
       try {
-        e = through_ring(*r, parts, n, stream);
+        e = through_ring(*r, staged, nstaged, stream);
       } catch (const std::bad_alloc&) {  // from the lists, before any thread is started
         e = hipErrorOutOfMemory;
       }
       (void)hipStreamSynchronize(stream);  // nothing is on its way into the ring when it is given back
       give_ring(r);
-      if (e == hipSuccess) return e;
+      arrived = e == hipSuccess;
     }
   }
   for (int p = 0; p < n; p++) {
+    if (arrived && !known(parts[p].dst)) continue;
     const hipError_t e = hipMemcpyAsync(parts[p].dst, parts[p].src, parts[p].bytes, hipMemcpyDeviceToHost, stream);
     if (e != hipSuccess) return e;
   }

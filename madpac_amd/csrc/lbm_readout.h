@@ -1,4 +1,4 @@
-// Device-to-host copies of results into the caller's (pageable) memory.
+// Device-to-host copies of results into the caller's memory.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -1,9 +1,10 @@
 // Host-only driver of the large readouts (madpac_amd/csrc/lbm_readout.cpp) over a stand-in for the few
 // runtime calls they make: "device" memory is host memory and copies happen at once.
 //
-// usage: test_readout whole | nothreads K
+// usage: test_readout whole | nothreads K | known
 //   whole        parts around the switch to the ring and with ragged last pieces arrive whole
 //   nothreads K  creating a thread runs out of memory after K of them were started
+//   known        parts in memory that the runtime knows (pinned) are copied there directly, others not
 #include <dlfcn.h>
 #include <pthread.h>
 #include <stdlib.h>
@@ -22,6 +23,7 @@ thread_local bool g_out_of_memory = false;   // operator new of this thread fail
 int g_started = 0;
 std::atomic<size_t> g_direct{0};             // bytes that a copy moved straight into the caller's memory
 const char *g_user = nullptr, *g_user_end = nullptr;
+const char *g_known = nullptr, *g_known_end = nullptr;  // pinned memory
 }  // namespace
 
 void* operator new(size_t n) {
@@ -51,6 +53,11 @@ hipError_t hipEventDestroy(hipEvent_t e) { return free((void*)e), hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+  std::memset(a, 0, sizeof(*a));
+  a->type = (const char*)p >= g_known && (const char*)p < g_known_end ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
+  return hipSuccess;
+}
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t) {
   std::memcpy(dst, src, n);
   if ((const char*)dst >= g_user && (const char*)dst < g_user_end) g_direct += n;
@@ -59,8 +66,9 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, h
 }
 
 namespace {
-// `sizes` bytes from as many sources into one destination; whether every byte arrived and nothing else changed
-bool arrives(const std::vector<size_t>& sizes) {
+// `sizes` bytes from as many sources into one destination, part `pinned` into pinned memory; whether every byte
+// arrived and nothing else changed
+bool arrives(const std::vector<size_t>& sizes, int pinned = -1) {
   size_t total = 0;
   for (size_t s : sizes) total += s;
   std::vector<unsigned char> src(total), dst(total + 64, 0xA5);
@@ -70,6 +78,10 @@ bool arrives(const std::vector<size_t>& sizes) {
   size_t o = 0;
   for (size_t s : sizes) {
     parts.push_back(lbm::HostCopy{dst.data() + o, src.data() + o, s});
+    if ((int)parts.size() - 1 == pinned) {
+      g_known = (const char*)dst.data() + o;
+      g_known_end = g_known + s;
+    }
     o += s;
   }
   g_user = (const char*)dst.data();
@@ -98,6 +110,11 @@ int main(int argc, char** argv) {
     ok = arrives({40 * MB + 24}) && g_started == atoi(argv[2]);
     g_allowed = -1;
     ok = ok && arrives({40 * MB + 24});
+  } else if (argc == 2 && !std::strcmp(argv[1], "known")) {
+    ok = arrives({32 * MB + 8}, 0) && g_direct == 32 * MB + 8;
+    ok = ok && arrives({30 * MB, 30 * MB + 16}, 0) && g_direct == 30 * MB;
+    ok = ok && arrives({30 * MB, 30 * MB + 16}, 1) && g_direct == 30 * MB + 16;
+    ok = ok && arrives({8 * MB, 23 * MB, 8}, 0) && g_direct == 31 * MB + 8;  // the rest is below the switch
   }
   lbm::readout_release();
   std::printf("%s\n", ok ? "ok" : "failed");

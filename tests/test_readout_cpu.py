@@ -31,3 +31,7 @@ def test_parts_arrive_whole(exe):
 def test_running_out_of_memory_between_threads(exe, started):
     # the threads that were started move every piece; the process goes on
     _run(exe, "nothreads", str(started))
+
+
+def test_memory_that_the_runtime_knows_is_copied_to_directly(exe):
+    _run(exe, "known")
