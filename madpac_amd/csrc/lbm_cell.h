@@ -250,8 +250,9 @@ __device__ __forceinline__ float collide_f32s(float (&g)[Q], const CollideParams
 // viscosity by up to ~1e-6 relative near tau = 0.5, where nu = (1/omega - 1/2) / 3 is small.
 // Against an all-FP64 evaluation of the same update (widen, collide, round once at the store) it
 // holds fewer FP64 values live: 60 instead of 76 VGPRs in the dense step, 8 instead of 6 waves per
-// SIMD, +6 % throughput.  Outputs as collide_f32s.
-template <bool FORCE, bool ALPHA>
+// SIMD, +6 % throughput.  Outputs as collide_f32s.  MIRROR: a direction and its mirror share their
+// quadratic terms (the same bits either way).
+template <bool FORCE, bool ALPHA, bool MIRROR = true>
 __device__ __forceinline__ float collide_f32s_h(float (&gs)[Q], const CollideParams& p, const CollideParams32& p32,
                                                 float alpha, float (&uo)[4]) {
   double drho = 0.0, j0 = 0.0, j1 = 0.0, j2 = 0.0;
@@ -292,14 +293,25 @@ __device__ __forceinline__ float collide_f32s_h(float (&gs)[Q], const CollidePar
     if (FORCE) v += p32.fpref * W32(q) * rho32 * (3.0f * (cg - ug) + quad);
     gs[q] = v;
   };
+  auto c_g = [&](int q) {
+    return FORCE ? (float)CX(q) * p32.g[0] + (float)CY(q) * p32.g[1] + (float)CZ(q) * p32.g[2] : 0.f;
+  };
+  if constexpr (!MIRROR) {
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      const double cu = cdot64(q, u0, u1, u2);
+      const float cg = c_g(q);
+      relax(q, 3.0 * cu + 4.5 * cu * cu - uu15, cg, FORCE ? 9.0f * (float)cu * cg : 0.f);
+    }
+    return rho32;
+  }
   relax(REST, 0.0 - uu15, 0.f, 0.f);
 #pragma unroll
   for (int q = 0; q < REST; q++) {
-    // a direction and its mirror: c.u and c.g change sign, the quadratic terms are shared (exactly)
+    // c.u and c.g change sign, the quadratic terms are shared (exactly)
     const double cu = cdot64(q, u0, u1, u2);
     const double a = 3.0 * cu, b = 4.5 * cu * cu;
-    const float cg = FORCE ? (float)CX(q) * p32.g[0] + (float)CY(q) * p32.g[1] + (float)CZ(q) * p32.g[2] : 0.f;
-    const float quad = FORCE ? 9.0f * (float)cu * cg : 0.f;
+    const float cg = c_g(q), quad = FORCE ? 9.0f * (float)cu * cg : 0.f;
     relax(q, a + b - uu15, cg, quad);
     relax(Q - 1 - q, -a + b - uu15, -cg, quad);
   }

@@ -9,7 +9,7 @@ namespace lbm {
 // Collision of one fluid cell plus the boundary classes of its bounce-back links (shared by the
 // two-buffer and the AA steps).  T = double: reference arithmetic; T = float: shifted populations,
 // hybrid arithmetic (collide_f32s_h) unless M32 (all FP32).
-template <typename T, bool FORCE, bool ALPHA, bool WALLS, bool M32>
+template <typename T, bool FORCE, bool ALPHA, bool WALLS, bool M32, bool MIRROR = true>
 __device__ __forceinline__ void collide_cell_bc(T (&f)[Q], uint32_t w, int64_t i, const T* __restrict__ alpha,
                                                 const CollideParams& p64, const CollideParams32& p32,
                                                 const BoundaryArgs& bc) {
@@ -21,7 +21,7 @@ __device__ __forceinline__ void collide_cell_bc(T (&f)[Q], uint32_t w, int64_t i
   } else if constexpr (M32) {
     rho = collide_f32s<FORCE, ALPHA>(f, p32, a, uc);
   } else {
-    rho = collide_f32s_h<FORCE, ALPHA>(f, p64, p32, a, uc);
+    rho = collide_f32s_h<FORCE, ALPHA, MIRROR>(f, p64, p32, a, uc);
   }
   if (WALLS) {
     const uint32_t k = (w >> CLASS_SHIFT) & CLASS_BITS;

@@ -15,8 +15,6 @@
 // BLB/nonlocaltreatment/AABlockStreaming.cpp:19-92); storing the post-collision state and
 // pulling gives the same numbers, because a moving-wall correction is applied to the outgoing
 // population of a wall link, which only that cell's own bounce-back ever reads.
-#include <type_traits>
-
 #include "lbm_collide.h"
 #include "lbm_geom.h"
 
@@ -98,12 +96,24 @@ __global__ __launch_bounds__(BX * BY_MAX) void k_build_words(DenseGeom g, const 
 }
 
 // ------------------------------------------------------------------------------------------
+// A kernel that holds both kinds of store (state_cached) is scheduled anew by the compiler, for the worse on
+// lattices that wait for latency.  The in-place step has one kind per kernel (with both, FP32 lid 30^3 5.14
+// us a step, 64 x 40 x 40 7.32; with one 4.99 and 7.12; 100^3 FP64 65.8 and 64.0).  The two-buffer step does so
+// (STREAM) on FP32 lattices of up to 1.5 wavefronts a SIMD: both / one kind 30 x 32 x 31 force 5.21 / 4.96, 44 x
+// 40 x 42 force 6.83 / 6.46; above and in FP64 both are no worse and often better (FP32 60^3 force 10.9 / 11.3;
+// FP64 44 x 43 x 45 lid 8.4 / 9.0).
+constexpr int64_t STREAM_CELLS = 3 * 64 * 4 * 256 / 2;  // 1.5 wavefronts on each of the 256 CUs' four SIMDs
+static bool stream_only(const DenseGeom& g, bool fp32) { return fp32 && g.Nu <= STREAM_CELLS && !g.cached; }
+
 // The hot kernel.  T = double: reference arithmetic; T = float: shifted populations.
 // SPEC = false: the flag word is read first, then the 19 loads at the pulled addresses (two
 // dependent memory round trips; solid lanes load nothing).  SPEC = true: the 19 neighbour loads
 // issue together with the word, and the few bounce-back populations are re-loaded from the cell's
 // own reflected slots once the word has arrived (one round trip on most lanes; solid lanes load).
-template <typename T, bool FORCE, bool ALPHA, bool WALLS, bool SPEC, bool M32, bool AOS>
+// On rows that are not interleaved, the FP32 collision without a force (or on small lattices) shares no terms
+// between mirrored directions: where it does, the compiler waits for loads in the middle of their chain
+// (30 x 32 x 31 periodic 4.87 us a step, 4.58 without; 50 x 49 x 51 7.9 and 7.6; with a force 60^3 10.9 and 12.0).
+template <typename T, bool FORCE, bool ALPHA, bool WALLS, bool SPEC, bool M32, bool AOS, bool STREAM>
 __global__ __launch_bounds__(BX * BY_MAX) void k_dense_step(DenseGeom g, const T* __restrict__ src,
                                                         T* __restrict__ dst, const uint32_t* __restrict__ words,
                                                         const T* __restrict__ alpha, CollideParams p64,
@@ -126,7 +136,7 @@ __global__ __launch_bounds__(BX * BY_MAX) void k_dense_step(DenseGeom g, const T
         for (int q = 0; q < Q; q++)
           if ((w >> (Q - 1 - q)) & 1u) f[q] = src[A.own(Q - 1 - q)];
       }
-      collide_cell_bc<T, FORCE, ALPHA, WALLS, M32>(f, w, c.i, alpha, p64, p32, bc);
+      collide_cell_bc<T, FORCE, ALPHA, WALLS, M32, AOS || (FORCE && !STREAM)>(f, w, c.i, alpha, p64, p32, bc);
     } else {
 #pragma unroll
       for (int q = 0; q < Q; q++) f[q] = T(0);
@@ -139,13 +149,13 @@ __global__ __launch_bounds__(BX * BY_MAX) void k_dense_step(DenseGeom g, const T
     if (fl) {
 #pragma unroll
       for (int q = 0; q < Q; q++) f[q] = src[((w >> (Q - 1 - q)) & 1u) ? A.own(Q - 1 - q) : A.pull(q)];
-      collide_cell_bc<T, FORCE, ALPHA, WALLS, M32>(f, w, c.i, alpha, p64, p32, bc);
+      collide_cell_bc<T, FORCE, ALPHA, WALLS, M32, AOS || (FORCE && !STREAM)>(f, w, c.i, alpha, p64, p32, bc);
     } else {
 #pragma unroll
       for (int q = 0; q < Q; q++) f[q] = T(0);
     }
   }
-  if (g.cached) {
+  if (!STREAM && g.cached) {
     asm volatile("");
 #pragma unroll
     for (int q = 0; q < Q; q++) dst[A.own(q)] = f[q];
@@ -165,7 +175,7 @@ __global__ __launch_bounds__(BX * BY_MAX) void k_dense_step(DenseGeom g, const T
 // cell writes exactly the slots it read, and no other cell touches them, so the update is in place
 // without races.  Boundary classes act on the outgoing population of a bounce-back link, as in the
 // two-buffer step.
-template <typename T, bool FORCE, bool ALPHA, bool WALLS, bool M32, bool ODD, bool AOS>
+template <typename T, bool FORCE, bool ALPHA, bool WALLS, bool M32, bool ODD, bool AOS, bool CACHED>
 __global__ __launch_bounds__(BX * BY_MAX) void k_aa_step(DenseGeom g, T* __restrict__ a, const uint32_t* __restrict__ words,
                                                      const T* __restrict__ alpha, CollideParams p64,
                                                      CollideParams32 p32, BoundaryArgs bc) {
@@ -194,25 +204,16 @@ __global__ __launch_bounds__(BX * BY_MAX) void k_aa_step(DenseGeom g, T* __restr
   // addresses live through the collision (38 more VGPRs, one wave less per SIMD); an opaque copy
   // of the cell's base address makes it recompute them here instead.
   asm volatile("" : "+v"(A.base));
-  auto store = [&](auto cached) {
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-      // x + c_q is not fluid (a solid lane stores its zeros to its own slots)
-      const bool bounce = ((fl ? w : 0x7FFFFu) >> q) & 1u;
-      const int64_t di = (!ODD || bounce) ? A.own(Q - 1 - q) : A.push(q);
-      if constexpr (decltype(cached)::value) a[di] = f[q];
-      else __builtin_nontemporal_store(f[q], &a[di]);
-    }
-  };
   // An even step writes whole lines of its own slots.  An odd step's pushes fill each line from
   // up to four wavefronts: ordinary stores let L2 merge the parts before write-back (measured
   // 5-13 % faster on a porous 256^3 channel than streaming stores, which write each part out).
-  if (ODD || g.cached) {
-    asm volatile("");
-    store(std::true_type{});
-    asm volatile("");
-  } else {
-    store(std::false_type{});
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    // x + c_q is not fluid (a solid lane stores its zeros to its own slots)
+    const bool bounce = ((fl ? w : 0x7FFFFu) >> q) & 1u;
+    const int64_t di = (!ODD || bounce) ? A.own(Q - 1 - q) : A.push(q);
+    if (CACHED) a[di] = f[q];
+    else __builtin_nontemporal_store(f[q], &a[di]);
   }
 }
 
@@ -555,9 +556,13 @@ static hipError_t step_t(const DenseGeom& g, const void* src, void* dst, const u
   const T* a = (const T*)alpha;
   const T* sp = (const T*)src;
   T* dp = (T*)dst;
-#define LBM_STEP(F, A, W)                                                                                        \
-  hipLaunchKernelGGL((k_dense_step<T, F, A, W, SPEC, M32, AOS>), dense_grid(g), dense_block(g), 0, s, g, sp, dp, words, a, \
-                     p64, p32, bc)
+#define LBM_STEP_S(F, A, W, S)                                                                                     \
+  hipLaunchKernelGGL((k_dense_step<T, F, A, W, SPEC, M32, AOS, S>), dense_grid(g), dense_block(g), 0, s, g, sp, dp, \
+                     words, a, p64, p32, bc)
+#define LBM_STEP(F, A, W)                                      \
+  if (stream_only(g, FP32)) LBM_STEP_S(F, A, W, FP32); \
+  else LBM_STEP_S(F, A, W, false)
+  constexpr bool FP32 = sizeof(T) == 4;
   const int key = (force ? 4 : 0) | (alpha ? 2 : 0) | (walls ? 1 : 0);
   switch (key) {
     case 0: LBM_STEP(false, false, false); break;
@@ -570,6 +575,7 @@ static hipError_t step_t(const DenseGeom& g, const void* src, void* dst, const u
     default: LBM_STEP(true, true, true); break;
   }
 #undef LBM_STEP
+#undef LBM_STEP_S
   return hipGetLastError();
 }
 
@@ -600,9 +606,12 @@ static hipError_t aa_t(const DenseGeom& g, void* buf, const uint32_t* words, con
                        const CollideParams& p64, const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t s) {
   T* ap = (T*)buf;
   const T* al = (const T*)alpha;
-#define LBM_AA(F, A, W)                                                                                        \
-  hipLaunchKernelGGL((k_aa_step<T, F, A, W, M32, ODD, AOS>), dense_grid(g), dense_block(g), 0, s, g, ap, words, al, \
-                     p64, p32, bc)
+#define LBM_AA_C(F, A, W, C)                                                                                     \
+  hipLaunchKernelGGL((k_aa_step<T, F, A, W, M32, ODD, AOS, C>), dense_grid(g), dense_block(g), 0, s, g, ap, words, \
+                     al, p64, p32, bc)
+#define LBM_AA(F, A, W)                          \
+  if (ODD || g.cached) LBM_AA_C(F, A, W, true); \
+  else LBM_AA_C(F, A, W, ODD)
   const int key = (force ? 4 : 0) | (alpha ? 2 : 0) | (walls ? 1 : 0);
   switch (key) {
     case 0: LBM_AA(false, false, false); break;
@@ -615,6 +624,8 @@ static hipError_t aa_t(const DenseGeom& g, void* buf, const uint32_t* words, con
     default: LBM_AA(true, true, true); break;
   }
 #undef LBM_AA
+#undef LBM_AA_C
+#undef LBM_AA_S
   return hipGetLastError();
 }
 
