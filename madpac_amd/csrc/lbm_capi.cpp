@@ -509,7 +509,7 @@ StepPlan plan_steps(const lbm_ctx* c) {
   if (p.small) return p;
   bool open = false;
   for (const lbm::BoundaryClass& b : c->bct) open = open || (b.mask && (b.type & lbm::BC_TYPE_MASK) != lbm::BC_MOVING_WALL);
-  if (lbm::pair_plan(c->g, c->splits, c->esize, c->nfluid, c->force || c->alpha, c->walls, open,
+  if (lbm::pair_plan(c->g, c->splits, c->esize, c->f32math, c->nfluid, c->force || c->alpha, c->walls, open,
                      p.coupled ? c->ncboxes : 0, &p.pair))
     p.most = 2;
   return p;

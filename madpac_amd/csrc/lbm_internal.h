@@ -166,11 +166,11 @@ struct PairSplits {
 };
 PairSplits pair_splits(const DenseGeom& g);
 // The split that this lattice takes, and whether launch_dense_pair takes it and is the faster way.
-// extra: force or porosity; walls: boundary classes; open: classes other than moving walls; coupled_boxes: boxes that
+// f32math: FP32 arithmetic; extra: force or porosity; walls: boundary classes; open: classes other than moving walls; coupled_boxes: boxes that
 // launch_coupled_boxes has to follow with (0: no coupling).
 // nfluid: fluid cells.
-bool pair_plan(const DenseGeom& g, const PairSplits& splits, size_t esize, int64_t nfluid, bool extra, bool walls,
-               bool open, int coupled_boxes, PairGeom* plan);
+bool pair_plan(const DenseGeom& g, const PairSplits& splits, size_t esize, bool f32math, int64_t nfluid, bool extra,
+               bool walls, bool open, int coupled_boxes, PairGeom* plan);
 hipError_t launch_dense_pair(const DenseGeom& g, const PairGeom& plan, bool fp32, bool f32math, const void* src, void* dst,
                              const uint32_t* words, const void* alpha, bool force, bool walls, const CollideParams& p64,
                              const CollideParams32& p32, const BoundaryArgs& bc, hipStream_t stream);

@@ -358,12 +358,26 @@ PairSplits pair_splits(const DenseGeom& g) { return PairSplits{pair_geom(g, 64, 
 //    solid cells' bytes a half (where the caches hold them, none).
 //  * This kernel: its planes in sequence (PairGeom::passes), each a latency: loads, two collisions, two
 //    barriers.  Force, porosity and boundary classes lengthen the collisions, open boundaries most: their
-//    cells' two equilibria per link hold up the whole workgroup.
-// Measured per step, one-step / this kernel: FP32 96^3 periodic 25.9 / 29, lid 27.8 / 35, channel 30.5 / 47;
-// 112^3 35.6 / 37.5; 128^3 55.3 / 46.7, force and porosity 56.6 / 54.2; 192^3 187 / 167, channel 189 / 240; 256^3 458 /
-// 355, channel 502 / 530.  FP64 64^3 14.2 / 12.7, force and porosity 14.0 / 14.8, lid 15.3 / 14.7; 80^3 30.9 / 23.5,
-// channel 30.7 / 38; 131 x 70 x 53 31.8 / 21.8, channel 31.6 / 32.0; 256^3 932 / 527.  The microseconds of a plane
-// are this table's.
+//    cells' two equilibria per link hold up the whole workgroup.  Past the Infinity Cache (two states of 200 MB),
+//    the FP32 planes with force or porosity take longer (not with FP32 arithmetic), as FP64 ones with solids do.
+// Measured per step in long runs, one-step / this kernel, us:
+//               periodic       lid            channel *      porous *       porosity
+//   FP64 64^3   14.1 / 12.3    15.0 / 14.0    16.4 / 18.9    15.3 / 17.0    14.3 / 15.8     (* with a tenth of
+//   80^3        31.0 / 21.6    30.9 / 22.0    33.5 / 29.7    34.5 / 31.3    30.4 / 25.3      the cells solid, at
+//   131x70x53   31.4 / 21.5    32.5 / 24.9    36.4 / 33.2    36.8 / 32.8    32.6 / 28.7      random; porous: and
+//   128^3        111 / 74       113 / 76       117 / 91       112 / 93       114 / 82        a force)
+//   1000x1000x2  119 / 91       124 / 89       124 / 97       130 / 138      120 / 92
+//   240^3        820 / 502      816 / 520      843 / 643      838 / 640      838 / 590
+//   FP32 96^3   26.3 / 23.4    27.7 / 27.0    30.7 / 35.7    32.7 / 30.4    28.7 / 28.5
+//   112^3       37.2 / 35.8    42.8 / 43.4    47.3 / 58.3    51.3 / 48.1    45.7 / 46.3
+//   128^3       56.3 / 47.6    55.9 / 50.4    63.2 / 66.8    60.7 / 56.5    56.2 / 55.5
+//   192x192x96  93.4 / 87.9    93.0 / 89.6     101 / 119      100 / 106     94.4 / 100
+//   240^3        437 / 359      437 / 378      472 / 516      472 / 416      445 / 402
+// The microseconds of a plane follow from these and 550 other runs.  Of what the rule sends here, two are more than
+// 3 % slower than single steps: FP64 rows of 8 cells in a box of thousands of planes (8 x 8 x 8192 porous 112 /
+// 90 us; the idle lanes are overrated there) and FP64 porosity on 72^3 (27.0 / 26.1).  Runs that start from a
+// state in memory gain less: the forward sweep of the adjoint with its checkpoints takes on 128^3 FP32 59.7 us a step
+// here and 57.6 in single steps, 128^3 FP64 83 and 113, 160^3 FP32 118 and 128.
 //  * With the MD coupling this kernel is followed by the boxes around the coupled cells (lbm_small.hip): 16 us
 //    and 45 ns a box (96^3 FP64: 14 us for 8 boxes, 23 for 216, 35 for 512, 173 for 3294), where a single step
 //    is followed by its re-collision, 7.5 us.  Per step, single / this way: 96^3 FP64 24^3 coupled cells 66.5 /
@@ -373,8 +387,8 @@ PairSplits pair_splits(const DenseGeom& g) { return PairSplits{pair_geom(g, 64, 
 //    empty at their end.  A step in 64 x 8 / 32 x 16: FP64 80^3 force and porosity 30.8 / 24.4, 96^3 (13 and 10
 //    planes) lid 40.0 / 34.5, channel 50.9 / 42.3, 160^3 (43 and 35) 155 / 145; FP32 160^3 118 / 105.
 // A plane of populations has to fit the 32-bit offsets.
-bool pair_plan(const DenseGeom& g, const PairSplits& splits, size_t esize, int64_t nfluid, bool extra, bool walls,
-               bool open, int coupled_boxes, PairGeom* plan) {
+bool pair_plan(const DenseGeom& g, const PairSplits& splits, size_t esize, bool f32math, int64_t nfluid, bool extra,
+               bool walls, bool open, int coupled_boxes, PairGeom* plan) {
   const int64_t plane = g.bricked ? (int64_t)64 * g.bnx * g.bny : (int64_t)g.nx * g.ny;
   if (plane * (g.aos ? Q : 1) * (int64_t)esize > (int64_t)UINT32_MAX) return false;
   const bool f64 = esize == 8;
@@ -382,14 +396,16 @@ bool pair_plan(const DenseGeom& g, const PairSplits& splits, size_t esize, int64
   const bool bricks = f64 && g.bricked;
   const double t_wide = (double)wide.passes * (bricks ? 1.04 : 1.0), t_tall = (double)tall.passes * (bricks ? 1.0 : 1.05);
   *plan = t_tall < t_wide ? tall : wide;
-  const bool held = g.cached && (double)Q * (double)g.N * (double)esize <= 125e6;
+  const double bytes = (double)Q * (double)g.N * (double)esize;
+  const bool held = g.cached && bytes <= 125e6;
   double cells = held ? (double)nfluid : 0.5 * ((double)nfluid + (double)g.Nu);
   if (!g.bricked) {
     cells *= 0.5 + 0.5 * ((g.nx + 63) / 64 * 64) / g.nx;
     if ((g.nx * esize) % 128) cells *= 1.2;
   }
   const double step = 3.0 + (walls ? 1.0 : 0.0) + cells * 2 * Q * (double)esize / (held ? 7.0e6 : 5.3e6);
-  const double pass = open ? (f64 ? 8.0 : 8.5) : extra ? (f64 ? 6.2 : 5.7) : walls ? (f64 ? 5.9 : 5.7) : (f64 ? 5.2 : 5.1);
+  const double more = f64 ? (nfluid < g.Nu && !held ? 6.8 : 6.2) : (!f32math && bytes > 200e6 ? 6.5 : 5.7);
+  const double pass = open ? (f64 ? 8.0 : 8.5) : extra ? more : walls ? (f64 ? 5.9 : 5.7) : (f64 ? 5.2 : 5.1);
   const double two = std::min(t_wide, t_tall) * pass;
   return coupled_boxes ? two + 16.0 + 0.045 * coupled_boxes < 2.0 * (step + 7.5) : two < 2.0 * step;
 }
