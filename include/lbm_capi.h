@@ -176,6 +176,12 @@ int lbm_get_populations(lbm_ctx* ctx, double* f);
 /* nsteps fused collide+stream steps: phases A, B and C of one reference iteration
  * (BLB/mappings/RegularGrid2RegularBlockSolver.cpp:83-248) per step. */
 int lbm_step(lbm_ctx* ctx, int nsteps);
+/* How lbm_step cuts a run of steps into launches on the context as it stands: the most steps that one
+ * launch takes, 1 (in place always), 2 (two-step kernel), or up to 4 on small lattices; *tile_x (may be
+ * NULL) receives the width of the two-step kernel's tiles, 64 (of 64 x 8 columns) or 32 (of 32 x 16),
+ * else 0.  LBM_ERR_STATE before lbm_set_flags.  The state is the same bits either way; for measurement
+ * and tests. */
+int lbm_step_plan(lbm_ctx* ctx, int* tile_x);
 /* Same steps, replayed from a hipGraph of 32 steps captured on the first call (one graph per
  * starting buffer or AA parity; the remainder runs as plain steps).  Anything the launches bake in
  * (cell order, porosity, per-cell velocities, wall classes present, body force, load schedule, MD

@@ -627,6 +627,14 @@ int lbm_step(lbm_ctx* c, int nsteps) {
   return lbm_enqueue_steps(c, nsteps);
 }
 
+int lbm_step_plan(lbm_ctx* c, int* tile_x) {
+  if (!c) return LBM_ERR_ARG;
+  if (!c->flags_set) return fail(c, LBM_ERR_STATE, "boundary flags not set (lbm_set_flags)");
+  const StepPlan p = c->aa ? StepPlan{} : plan_steps(c);
+  if (tile_x) *tile_x = p.most == 2 && !p.small ? p.pair.tile_x : 0;
+  return p.most;
+}
+
 int lbm_step_graph(lbm_ctx* c, int nsteps) {
   if (!c) return LBM_ERR_ARG;
   if (nsteps < 0) return fail(c, LBM_ERR_ARG, "nsteps must be >= 0");

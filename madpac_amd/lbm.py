@@ -40,7 +40,8 @@ EXPORTS = (
     "lbm_set_boundary_class", "lbm_set_moving_wall_class", "lbm_set_wall_classes", "lbm_set_boundary_velocity",
     "lbm_set_cavity_lid", "lbm_set_channel", "lbm_set_porosity",
     "lbm_set_coupling_cells", "lbm_set_coupling_data", "lbm_get_coupling_data",
-    "lbm_init_equilibrium", "lbm_set_populations", "lbm_get_populations", "lbm_step", "lbm_step_timed", "lbm_measure_copy",
+    "lbm_init_equilibrium", "lbm_set_populations", "lbm_get_populations", "lbm_step", "lbm_step_plan", "lbm_step_timed",
+    "lbm_measure_copy",
     "lbm_tune", "lbm_synchronize", "lbm_get_fields", "lbm_reduce_moments", "lbm_reduce_moments_noalloc",
     "lbm_kinetic_energy",
     "lbm_pressure_drop",
@@ -138,6 +139,7 @@ def load_library(path: str = LIB_PATH):
     L.lbm_set_populations.argtypes = [vp, dp]
     L.lbm_get_populations.argtypes = [vp, dp]
     L.lbm_step.argtypes = [vp, ctypes.c_int]
+    L.lbm_step_plan.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
     L.lbm_step_graph.argtypes = [vp, ctypes.c_int]
     L.lbm_step_timed.argtypes = [vp, ctypes.c_int, ctypes.POINTER(ctypes.c_float)]
     L.lbm_measure_copy.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_float)]
@@ -362,6 +364,14 @@ class Lattice:
             self._check(self._L.lbm_step_graph(self._h, int(n)), "lbm_step_graph")
         else:
             self._check(self._L.lbm_step(self._h, int(n)), "lbm_step")
+
+    def step_plan(self):
+        """(steps, tile_x) of the launches that step() makes of a long run: the most steps in one launch and
+        the width of the two-step kernel's tiles (64 or 32; 0 where another kernel runs)."""
+        tile = ctypes.c_int()
+        rc = self._L.lbm_step_plan(self._h, ctypes.byref(tile))
+        self._check(min(rc, 0), "lbm_step_plan")
+        return rc, int(tile.value)
 
     def step_timed(self, n):
         ms = ctypes.c_float()
