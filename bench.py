@@ -45,11 +45,6 @@ def read_traffic(key):
     return None
 
 
-def steps_per_launch(lbm, n, layout, steps):
-    """Two-buffer lattices of 128^3 cells and more without open boundaries advance two steps per launch."""
-    return 2 if layout == lbm.LAYOUT_TWO_BUFFER and steps >= 2 and n >= 128 else 1
-
-
 def run_dense(lbm, solid, n, tau, prec, steps, warmup, g, layout=0, readout=False):
     lat = lbm.Lattice(n, n, n, tau, precision=prec, periodic=(True, True, True), force=(g, 0.0, 0.0), layout=layout)
     lat.set_flags(~solid)
@@ -75,6 +70,7 @@ def run_dense(lbm, solid, n, tau, prec, steps, warmup, g, layout=0, readout=Fals
             cms = lat.measure_copy(steps, pull=pull) / steps
             ceil[key] = {"ms": round(cms, 4), "GBs": round(cells * 38 * esize_ / (cms * 1e-3) / 1e9, 1)}
     m = lat.moments()
+    per_launch = min(lat.step_plan()[0], steps)
     host = None
     if readout:  # what a caller pays to bring results to the host (PCIe), outside the timed steps
         t0 = time.perf_counter()
@@ -86,10 +82,9 @@ def run_dense(lbm, solid, n, tau, prec, steps, warmup, g, layout=0, readout=Fals
                 "populations_s": round(t2 - t1, 4), "populations_bytes": n ** 3 * 19 * 8}
     lat.close()
     esize = 8 if prec == lbm.FP64 else 4
-    # The two-buffer lattice of this size runs two steps per launch: one read and one write of the state for both.
+    # Where the lattice runs two steps per launch, there is one read and one write of the state for both.
     # `achieved` counts the bytes that a launch has to move; `one_step` the 38 values of every update, which a
     # one-step kernel would have to move (it can exceed what HBM carries).
-    per_launch = steps_per_launch(lbm, n, layout, steps)
     bytes_per_launch = nfluid * 2 * 19 * esize
     achieved = bytes_per_launch / (ms * 1e-3 / steps * per_launch) / 1e9
     schedule = "aa-in-place" if layout == lbm.LAYOUT_AA else ("loads-with-flag-word" if variant & 1 else "flag-word-first")
@@ -171,8 +166,8 @@ def run_taylor_green(lbm, wl, n=512, steps=200, tau=0.52, u0=0.04):
             lat.tune(20)
             lat.step(10)
             ms = lat.step_timed(steps) / steps
+            k = min(lat.step_plan()[0], steps)
         esize = 8 if prec == lbm.FP64 else 4
-        k = steps_per_launch(lbm, n, lbm.LAYOUT_TWO_BUFFER, steps)
         gbs = n ** 3 * 38 * esize / (k * ms * 1e-3) / 1e9  # the state read and written once per launch
         out[name] = {"value": round(n ** 3 / (ms * 1e3), 1), "unit": "MLUPS", "ms_per_step": round(ms, 4),
                      "steps_per_launch": k, "roofline_frac": round(gbs / HBM_PEAK_GBS, 4)}
@@ -196,10 +191,11 @@ def run_shard_share(lbm, solid, tau, g, planes=32, steps=300):
             ms = lat.step_timed(steps) / steps
             nfl = lat.fluid_cells
             order = "bricks" if lat.cell_order == lbm.CELL_ORDER_BRICKS else "rows"
+            k = min(lat.step_plan()[0], steps)
         esize = 8 if prec == lbm.FP64 else 4
         out[name] = {"value": round(nfl / (ms * 1e3), 1), "unit": "MLUPS", "ms_per_step": round(ms, 4),
-                     "steps_per_launch": 2,  # 2.2 M cells: two steps per launch in both precisions
-                     "roofline_frac": round(nfl * 38 * esize / (2 * ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+                     "steps_per_launch": k,
+                     "roofline_frac": round(nfl * 38 * esize / (k * ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                      "cell_order": order}
     return out
 
