@@ -606,11 +606,14 @@ void graph_release(lbm_ctx* c, int slot) {
 }
 }  // namespace
 
-// Steps per captured graph (even).  Measured per step on MI355X / ROCm 7.2 (cavity 16^3 / 32^3 /
-// 64^3, plain launches 6.1 / 6.2 / 18.4 us): 2-step graphs 8.6 / 8.7 / 21.1 us, 8-step 6.6 / 6.8 /
-// 19.1 us, 32-step 7.0 / 6.4 / 18.6 us, 128-step 6.8 / 6.3 / 18.7 us.  Dependent kernels are bound by
-// the dispatch-to-dispatch latency either way; replays never beat plain launches here.
+// Steps per captured graph where a launch takes one or two: a multiple of four, as a graph has to hold an even
+// number of launches (the state must end in the buffer that the next replay starts from).  Small lattices
+// capture 12 launches.  Measured per step on MI355X / ROCm 7.2 in single steps (cavity 16^3 / 32^3 / 64^3, plain
+// launches 6.1 / 6.2 / 18.4 us): 2-step graphs 8.6 / 8.7 / 21.1 us, 8-step 6.6 / 6.8 / 19.1 us, 32-step 7.0 / 6.4 /
+// 18.6 us, 128-step 6.8 / 6.3 / 18.7 us.  Dependent kernels are bound by the dispatch-to-dispatch latency
+// either way; replays never beat plain launches here.
 constexpr int GRAPH_STEPS = 32;
+static_assert(GRAPH_STEPS % 4 == 0, "an even number of launches of one or two steps");
 
 void lbm_graphs_release(lbm_ctx* c) {
   for (int s = 0; s < 2; s++) graph_release(c, s);
@@ -645,13 +648,17 @@ int lbm_step_graph(lbm_ctx* c, int nsteps) {
   // an even number of launches, so that cur (or parity) ends at this slot's phase
   const int most = c->aa ? 1 : plan_steps(c).most, K = most > 2 ? 12 * most : GRAPH_STEPS;
   if (nsteps >= K) {
-    const lbm_graph_key key = graph_key(c);
+    lbm_graph_key key = graph_key(c);
+    key.steps = K;
     if (!c->gexec[slot] || !(c->gkey[slot] == key)) {
       graph_release(c, slot);
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
       rc = lbm_enqueue_steps(c, K);
       hipGraph_t g = nullptr;
       const hipError_t e = hipStreamEndCapture(c->stream, &g);
+      int& phase = c->aa ? c->parity : c->cur;
+      if (!rc && e == hipSuccess && phase != slot) rc = fail(c, LBM_ERR_STATE, "a captured run ends in the other phase");
+      phase = slot;  // nothing has run yet
       if (rc) {
         if (g) (void)hipGraphDestroy(g);
         return rc;

@@ -13,17 +13,17 @@ namespace lbm {
 struct AdjointState;  // lbm_adjoint.hip
 }
 
-// What a captured pair of steps bakes into its launches (besides fixed buffers and parameters):
+// What a captured run of `steps` steps bakes into its launches (besides fixed buffers and parameters):
 // a change of any of these re-captures the graph (lbm_step_graph).
 struct lbm_graph_key {
-  int bricked = -1, remap = -1, by = -1, walls = 0, force = 0, spec = 0, couple_on = 0, couple_mode = 0,
+  int steps = 0, bricked = -1, remap = -1, by = -1, walls = 0, force = 0, spec = 0, couple_on = 0, couple_mode = 0,
       couple_rho = 0;
   double couple_dt = 0.0;
   const void *alpha = nullptr, *bcu = nullptr, *ccells = nullptr, *cu = nullptr, *crho = nullptr, *csave = nullptr;
   int64_t ncouple = 0;
   bool operator==(const lbm_graph_key& o) const {
-    return bricked == o.bricked && remap == o.remap && by == o.by && walls == o.walls && force == o.force && spec == o.spec &&
-           couple_on == o.couple_on && couple_mode == o.couple_mode && couple_rho == o.couple_rho &&
+    return steps == o.steps && bricked == o.bricked && remap == o.remap && by == o.by && walls == o.walls &&
+           force == o.force && spec == o.spec && couple_on == o.couple_on && couple_mode == o.couple_mode && couple_rho == o.couple_rho &&
            couple_dt == o.couple_dt && alpha == o.alpha && bcu == o.bcu && ccells == o.ccells && cu == o.cu &&
            crho == o.crho && csave == o.csave && ncouple == o.ncouple;
   }
@@ -75,7 +75,7 @@ struct lbm_ctx {
   size_t scratch_bytes = 0;
   int64_t nfluid = 0;
   lbm::AdjointState* adj = nullptr;
-  // lbm_step_graph: two steps captured per starting phase (buffer `cur`, or the AA parity)
+  // lbm_step_graph: a run of steps captured per starting phase (buffer `cur`, or the AA parity)
   hipGraph_t graph[2] = {nullptr, nullptr};
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   lbm_graph_key gkey[2];
