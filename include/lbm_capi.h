@@ -207,7 +207,10 @@ int lbm_measure_copy(lbm_ctx* ctx, int mode, int nsteps, float* ms);
  * dispatch over the XCDs; 1 = each XCD a contiguous range of the lattice.  Bits 2-3, the workgroup
  * shape: 0 = the default (4 rows of 64 cells, or 4 bricks), 1/2/3 = 2/4/8 rows or bricks; the
  * timing covers the three explicit shapes.  Which is
- * faster depends on lattice size, cell order and allocation.  With nsteps == 0, *variant (0..15) is
+ * faster depends on lattice size, cell order and allocation.  Where lbm_step takes several steps per
+ * launch (lbm_step_plan), those launches are timed too, and the context keeps to single steps if the
+ * fastest variant beats them, as long as the fluid cells, the kinds of boundary class, the presence of a
+ * porosity and the coupled cells are the same; else the variant is that of the single steps which remain.  With nsteps == 0, *variant (0..15) is
  * an input and selects directly.  When the state copy does not fit the device, the current choice
  * is kept.  All variants give bit-identical states, and the reductions run with one fixed shape.
  * No reference counterpart. */
