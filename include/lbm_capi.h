@@ -182,18 +182,20 @@ int lbm_step(lbm_ctx* ctx, int nsteps);
  * else 0.  LBM_ERR_STATE before lbm_set_flags.  The state is the same bits either way; for measurement
  * and tests. */
 int lbm_step_plan(lbm_ctx* ctx, int* tile_x);
-/* Same steps, replayed from a hipGraph of 32 steps captured on the first call (one graph per
+/* Same steps, replayed from a hipGraph of 32 steps (48 or 36 on small lattices: 12 launches of four or
+ * three) captured on the first call (one graph per
  * starting buffer or AA parity; the remainder runs as plain steps).  Anything the launches bake in
- * (cell order, porosity, per-cell velocities, wall classes present, body force, load schedule, MD
+ * (steps per launch, cell order, porosity, per-cell velocities, wall classes present, body force, load schedule, MD
  * coupling) is checked on every call and a change re-captures.  Results are bit-identical to
  * lbm_step, whose launches are capture-safe (no memsets, copies or synchronisation).  On MI355X /
  * ROCm 7.2 replays are not faster than plain launches (both bound by the dispatch latency of
- * dependent kernels, ~6 us per step on small lattices).  No reference counterpart. */
+ * dependent kernels, 5 to 6 us a launch).  No reference counterpart. */
 int lbm_step_graph(lbm_ctx* ctx, int nsteps);
 /* Same, timed with HIP events on the context stream; *ms = elapsed device time. */
 int lbm_step_timed(lbm_ctx* ctx, int nsteps, float* ms);
 /* Bandwidth reference of the step, no reference counterpart (measurement): nsteps launches of a
- * kernel with the step's grid, workgroup mapping and non-temporal stores that moves all 19 values
+ * kernel with the one-step kernel's grid, workgroup mapping and kind of store (past the caches, but for states of
+ * 20 to 140 MB, which stay in them from one step to the next) that moves all 19 values
  * of every stored cell (solid ones too) from the current state buffer into the other one, with no
  * flag word and no arithmetic: mode 0 the cell's own slots (a 19-plane copy), mode 1 the slots the
  * step pulls from (the all-fluid step's access pattern).  The state is left unchanged; *ms is the

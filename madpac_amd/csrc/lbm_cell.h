@@ -87,13 +87,15 @@ __device__ __forceinline__ double cdot64(int q, double v0, double v1, double v2)
 // and zl = z 2^-54, and the sum before its one rounding is within 0.75 2^-106 of the quotient, relative;
 // no quotient of two doubles by these c lies that close to a rounding boundary (a midpoint quotient
 // m/2 would need |2^53 X - m C| < 1 for odd integers m, C (< 4 where 4 divides C): never).  Zeros,
-// infinities, NaN and overflow follow the division; below 2^-960 the last bit may not, and every
-// caller adds the result to 1.  Two FP64 instructions each; the compiler's division takes ten and a
+// infinities, NaN and overflow follow the division; below 2^-960 the last bit may not.  The equilibria add the
+// result to 1.  Two FP64 instructions each; the compiler's division takes ten and a
 // quarter-rate reciprocal, and 40 of them made a cell's collision 675 instructions instead of 270.
 __device__ __forceinline__ double over_cs2(double x) { return __builtin_fma(3.0, x, x * 0x1.8p-53); }
 __device__ __forceinline__ double over_cs2x2(double x) { return __builtin_fma(1.5, x, x * 0x1.8p-54); }
 __device__ __forceinline__ double over_cs4x2(double x) { return __builtin_fma(4.5, x, x * 0x1.2p-52); }
-// (1.0/3.0)*(1.0/3.0) of the coupling's force term is half of the third constant: the same proof, z = 9
+// (1.0/3.0)*(1.0/3.0) of the coupling's force term is half of the third constant: the same proof, z = 9.  Its
+// result (c.u)^2 / cs4 multiplies c.g and is added to 3 (c - u).g, so an inexact last bit (|c.u| < 2^-480) can reach a
+// population only where those terms cancel to less than 2^-900 of c.g.
 __device__ __forceinline__ double over_cs4(double x) { return __builtin_fma(9.0, x, x * 0x1.2p-51); }
 
 // computeFeq (BLB/BlockComputeCellValues.cpp:14-20) of direction q (cu = c_q . u, du = u.u / (2 cs2))

@@ -257,7 +257,7 @@ __global__ __launch_bounds__(BX * BY_MAX) void k_dense_unpull(DenseGeom g, const
 
 // Bandwidth reference of the step (measurement, not part of a time step): every stored cell of the
 // lattice (fluid or not) moves its 19 values from src to dst with the step's grid, workgroup mapping
-// and non-temporal stores, and no flag word or arithmetic.  PULL = false: each cell copies its own
+// and kind of store (state_cached), and no flag word or arithmetic.  PULL = false: each cell copies its own
 // slots (the 19-plane copy); PULL = true: it reads the slots the step pulls from (x - c_q, wrapped on
 // periodic axes, clamped otherwise), i.e. the all-fluid step's memory pattern.
 template <typename T, bool PULL, bool AOS>
