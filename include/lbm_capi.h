@@ -210,9 +210,9 @@ int lbm_measure_copy(lbm_ctx* ctx, int mode, int nsteps, float* ms);
  * shape: 0 = the default (4 rows of 64 cells, or 4 bricks), 1/2/3 = 2/4/8 rows or bricks; the
  * timing covers the three explicit shapes.  Which is
  * faster depends on lattice size, cell order and allocation.  Where lbm_step takes several steps per
- * launch (lbm_step_plan), those launches are timed too, and the context keeps to single steps if the
- * fastest variant beats them, as long as the fluid cells, the kinds of boundary class, the presence of a
- * porosity and the coupled cells are the same; else the variant is that of the single steps which remain.  With nsteps == 0, *variant (0..15) is
+ * launch (lbm_step_plan), the variants apply to the single steps that remain (and to lbm_step(ctx, 1)); whether
+ * it does is a rule, not measured here: the first launches of the two-step kernel after lighter work are up to a
+ * fifth slower than those of a long run, so that a short timing picks the wrong way.  With nsteps == 0, *variant (0..15) is
  * an input and selects directly.  When the state copy does not fit the device, the current choice
  * is kept.  All variants give bit-identical states, and the reductions run with one fixed shape.
  * No reference counterpart. */

@@ -500,30 +500,17 @@ struct StepPlan {
   lbm::PairGeom pair;
 };
 
-lbm_plan_inputs plan_inputs(const lbm_ctx* c) {
-  lbm_plan_inputs in;
-  in.bricked = c->g.bricked != 0;
-  in.walls = c->walls;
-  for (const lbm::BoundaryClass& b : c->bct)
-    in.open = in.open || (b.mask && (b.type & lbm::BC_TYPE_MASK) != lbm::BC_MOVING_WALL);
-  in.porosity = c->alpha != nullptr;
-  in.ncouple = c->couple_on ? c->ncouple : 0;
-  in.coupled_boxes = in.ncouple ? c->ncboxes : 0;
-  in.nfluid = c->nfluid;
-  return in;
-}
-
 StepPlan plan_steps(const lbm_ctx* c) {
   StepPlan p;
-  const lbm_plan_inputs in = plan_inputs(c);
-  if (c->keep_single && in == c->tuned) return p;
-  p.coupled = in.ncouple != 0;
-  const bool extra = c->force || in.porosity;
-  if (p.coupled && (!in.coupled_boxes || extra)) return p;  // single steps, each with its re-collision
+  p.coupled = c->couple_on && c->ncouple;
+  if (p.coupled && (!c->ncboxes || c->force || c->alpha)) return p;  // single steps, each with its re-collision
   if (!p.coupled) p.most = lbm::small_steps(c->g);
   p.small = p.most > 1;
   if (p.small) return p;
-  if (lbm::pair_plan(c->g, c->splits, c->esize, c->f32math, in.nfluid, extra, in.walls, in.open, in.coupled_boxes, &p.pair))
+  bool open = false;
+  for (const lbm::BoundaryClass& b : c->bct) open = open || (b.mask && (b.type & lbm::BC_TYPE_MASK) != lbm::BC_MOVING_WALL);
+  if (lbm::pair_plan(c->g, c->splits, c->esize, c->f32math, c->nfluid, c->force || c->alpha, c->walls, open,
+                     p.coupled ? c->ncboxes : 0, &p.pair))
     p.most = 2;
   return p;
 }
@@ -663,7 +650,6 @@ int lbm_step_graph(lbm_ctx* c, int nsteps) {
   if (nsteps >= K) {
     lbm_graph_key key = graph_key(c);
     key.steps = K;
-    key.most = most;
     if (!c->gexec[slot] || !(c->gkey[slot] == key)) {
       graph_release(c, slot);
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -751,7 +737,6 @@ int lbm_tune(lbm_ctx* c, int nsteps, int* variant) {
   if (nsteps == 0) {  // explicit choice
     if (!variant || *variant < 0 || *variant > 15) return fail(c, LBM_ERR_ARG, "variant must be in 0..15");
     apply_variant(c, *variant);
-    c->keep_single = false;
     return LBM_OK;
   }
   int rc = need_state(c);
@@ -790,25 +775,6 @@ int lbm_tune(lbm_ctx* c, int nsteps, int* variant) {
     }
   }
   apply_variant(c, best_v);
-  // the launches of several steps that the rule plans, against the fastest variant (2 %: the noise of a timing)
-  c->keep_single = false;
-  const int most = c->aa ? 1 : plan_steps(c).most;
-  if (most > 1) {
-    const int n = (nsteps + most - 1) / most * most;
-    HIPCHK(c, hipMemcpyAsync(c->buf[cur0], c->scratch, bytes, hipMemcpyDeviceToDevice, c->stream));
-    c->cur = cur0;
-    rc = lbm_enqueue_steps(c, most);
-    if (rc) return rc;
-    float ms = 0.f;
-    HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    rc = lbm_enqueue_steps(c, n);
-    if (rc) return rc;
-    HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-    HIPCHK(c, hipEventSynchronize(c->ev1));
-    HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
-    c->keep_single = best / nsteps < 0.98f * ms / n;
-    c->tuned = plan_inputs(c);
-  }
   HIPCHK(c, hipMemcpyAsync(c->buf[cur0], c->scratch, bytes, hipMemcpyDeviceToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->cur = cur0;

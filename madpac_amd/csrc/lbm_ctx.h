@@ -16,27 +16,16 @@ struct AdjointState;  // lbm_adjoint.hip
 // What a captured run of `steps` steps bakes into its launches (besides fixed buffers and parameters):
 // a change of any of these re-captures the graph (lbm_step_graph).
 struct lbm_graph_key {
-  int steps = 0, most = 0, bricked = -1, remap = -1, by = -1, walls = 0, force = 0, spec = 0, couple_on = 0, couple_mode = 0,
+  int steps = 0, bricked = -1, remap = -1, by = -1, walls = 0, force = 0, spec = 0, couple_on = 0, couple_mode = 0,
       couple_rho = 0;
   double couple_dt = 0.0;
   const void *alpha = nullptr, *bcu = nullptr, *ccells = nullptr, *cu = nullptr, *crho = nullptr, *csave = nullptr;
   int64_t ncouple = 0;
   bool operator==(const lbm_graph_key& o) const {
-    return steps == o.steps && most == o.most && bricked == o.bricked && remap == o.remap && by == o.by && walls == o.walls &&
+    return steps == o.steps && bricked == o.bricked && remap == o.remap && by == o.by && walls == o.walls &&
            force == o.force && spec == o.spec && couple_on == o.couple_on && couple_mode == o.couple_mode && couple_rho == o.couple_rho &&
            couple_dt == o.couple_dt && alpha == o.alpha && bcu == o.bcu && ccells == o.ccells && cu == o.cu &&
            crho == o.crho && csave == o.csave && ncouple == o.ncouple;
-  }
-};
-
-// What the time of a step depends on beside its context's configuration.
-struct lbm_plan_inputs {
-  bool bricked = false, walls = false, open = false, porosity = false;  // open: classes other than moving walls
-  int coupled_boxes = 0;
-  int64_t ncouple = 0, nfluid = 0;  // ncouple: 0 while the coupling is off
-  bool operator==(const lbm_plan_inputs& o) const {
-    return bricked == o.bricked && walls == o.walls && open == o.open && porosity == o.porosity &&
-           coupled_boxes == o.coupled_boxes && ncouple == o.ncouple && nfluid == o.nfluid;
   }
 };
 
@@ -63,8 +52,6 @@ struct lbm_ctx {
   bool flags_set = false, state_set = false;
   bool walls = false, force = false;
   bool spec = false;                   // step-kernel load schedule (lbm_tune)
-  bool keep_single = false;            // lbm_tune measured single steps faster than the planned launches ...
-  lbm_plan_inputs tuned{};             // ... on this
   lbm::BoundaryClass bct[lbm::MAX_CLASSES]{};  // host copy of the boundary-class table
   lbm::BoundaryClass* d_bct = nullptr;          // device copy (read by the step kernels)
   double* d_bcu = nullptr;                      // per-cell target velocities [3*N] or null

@@ -381,8 +381,8 @@ class Lattice:
     def tune(self, nsteps=10, variant=None):
         """Pick the fastest step-kernel variant on the current state (returns 4..15: bit 0 the load
         schedule, bit 1 the XCD-contiguous workgroup order, bits 2-3 the workgroup shape 2/4/8 rows
-        or bricks), or with `variant` given (0..15; shape bits 0 = the default), select it.  Launches of
-        several steps (step_plan) are timed against it, and give way where it is faster."""
+        or bricks), or with `variant` given (0..15; shape bits 0 = the default), select it.  Where step()
+        takes several steps per launch (step_plan) it applies to the single steps that remain."""
         v = ctypes.c_int(0 if variant is None else int(variant))
         n = 0 if variant is not None else int(nsteps)
         self._check(self._L.lbm_tune(self._h, n, ctypes.byref(v)), "lbm_tune")
